@@ -80,7 +80,7 @@ typedef struct pf_plan_info {
     long long npts;
     int tile[3];
     long long spread_entries; /* (sample, tile) pairs of the spread list */
-    int spread_items;         /* work items of the finer split (batches with few value chunks) */
+    int spread_items;         /* work items of the split for batches of up to 16 values per point */
     int spread_slots;         /* partial tiles that split uses */
 } pf_plan_info;
 

@@ -35,7 +35,7 @@ struct pf_fft_cache;
 // footprint touches the tile, split into chunks of at most max_chunk entries.
 // Tiles with several chunks accumulate into partial tiles that a second
 // kernel sums in chunk order (deterministic).
-// spread work items over one sorted entry list
+// spread work items over one sorted entry list (pieces of pf_slist::items)
 struct pf_sitems {
     int4* sitems = nullptr;      // (key, e0, e1, slot or -1)
     int nsitems = 0;
@@ -49,24 +49,19 @@ struct pf_sitems {
     int nslots = 0;
 };
 
+constexpr int PF_NSPLIT = 4;
 constexpr int PF_SLIST_PAD = 16;  // readable ids past the end of a spread list
 
 struct pf_slist {
     int32_t* slist = nullptr;    // sorted sample ids grouped by key
     int64_t nslist = 0;
-    // [0] heavy tiles split; [1] split further so that the items alone fill
-    // the GPU; [2] as [1] with twice the item size, for batches of several
-    // value chunks (each item is then that many waves).  Arrays are shared
-    // where a split changes nothing.
-    pf_sitems split[3];
+    int4* items = nullptr;       // every split's items, one allocation
+    // heavy tiles split for batches of up to 8, 16, 32 and more values per
+    // grid point (pf_split_for); arrays are shared where the item size is
+    // the same
+    pf_sitems split[PF_NSPLIT];
 };
 
-// waves of a spread launch above which the coarser split is used: a batch
-// with several value chunks per tile fills the GPU without splitting tiles
-// further, and every extra split costs a partial tile per value chunk
-#ifndef PF_SPREAD_FILL
-#define PF_SPREAD_FILL 8192
-#endif
 #ifndef PF_COLMASK
 #define PF_COLMASK 1  // 3-D plans: skip the (y, x) grid columns no sample covers in the fused operators
 #endif
@@ -74,10 +69,9 @@ struct pf_slist {
 #define PF_SPREAD_MINCH 64  // smallest work item of the fine split (entries)
 #endif
 
-static inline const pf_sitems& pf_sitems_for(const pf_slist& L, int nvch) {
-    if ((int64_t)L.split[0].nsitems * nvch >= PF_SPREAD_FILL) return L.split[0];
-    return nvch > 1 ? L.split[2] : L.split[1];
-}
+static inline int pf_split_for(int V) { return V <= 8 ? 0 : (V <= 16 ? 1 : (V <= 32 ? 2 : 3)); }
+// work items of a batch of V values per grid point
+static inline const pf_sitems& pf_sitems_for(const pf_slist& L, int V) { return L.split[pf_split_for(V)]; }
 
 // Gather column lists (3-D plans with one kernel width on all axes): the
 // sorted samples regrouped by window key = (frame, y column, x column, z

@@ -204,8 +204,11 @@ __global__ void k_slist_count(const float* __restrict__ rec, TapParams P, uint32
     cnt[s] = n;
 }
 
-__global__ void k_slist_emit(const float* __restrict__ rec, TapParams P, int merge, const uint32_t* __restrict__ off,
-                             uint32_t* __restrict__ keys, int32_t* __restrict__ vals) {
+// key: (frame, tile) << sbits | position of the sample's first tap along the
+// slow axis sa relative to the tile (0 .. T + W - 2)
+__global__ void k_slist_emit(const float* __restrict__ rec, TapParams P, int merge, int sa, int sbits,
+                             const uint32_t* __restrict__ off, uint32_t* __restrict__ keys,
+                             int32_t* __restrict__ vals) {
     int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= P.mtot) return;
     const int* ri = reinterpret_cast<const int*>(rec + s * P.rec);
@@ -218,19 +221,25 @@ __global__ void k_slist_emit(const float* __restrict__ rec, TapParams P, int mer
     for (int a = 0; a < nz; ++a)
         for (int b = 0; b < ny; ++b)
             for (int c = 0; c < nx; ++c) {
-                keys[o] = (uint32_t)(f * P.ntile_tot + ((int64_t)tz[a] * P.ntiles[1] + ty[b]) * P.ntiles[2] + tx[c]);
+                uint32_t key = (uint32_t)(f * P.ntile_tot + ((int64_t)tz[a] * P.ntiles[1] + ty[b]) * P.ntiles[2] + tx[c]);
+                if (sbits) {
+                    int d = ri[sa] - (sa == 0 ? tz[a] : ty[b]) * P.tile[sa];
+                    if (d >= P.tile[sa]) d -= P.os[sa];  // a footprint entering the tile across the periodic edge
+                    key = (key << sbits) | (uint32_t)(d + P.width[sa] - 1);
+                }
+                keys[o] = key;
                 vals[o] = (int32_t)s;
                 ++o;
             }
 }
 
-__global__ void k_bounds(const uint32_t* __restrict__ keys, int64_t n, int32_t* __restrict__ start,
+__global__ void k_bounds(const uint32_t* __restrict__ keys, int64_t n, int sbits, int32_t* __restrict__ start,
                          int32_t* __restrict__ end) {
     int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    uint32_t k = keys[e];
-    if (e == 0 || keys[e - 1] != k) start[k] = (int32_t)e;
-    if (e == n - 1 || keys[e + 1] != k) end[k] = (int32_t)(e + 1);
+    const uint32_t k = keys[e] >> sbits;
+    if (e == 0 || keys[e - 1] >> sbits != k) start[k] = (int32_t)e;
+    if (e == n - 1 || keys[e + 1] >> sbits != k) end[k] = (int32_t)(e + 1);
 }
 
 // Window key of every sorted sample for the LDS-staged gather: (frame,
@@ -362,7 +371,14 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
     const int64_t M = p->mtot;
     const int TB = 256;
     const uint64_t nkeys = (uint64_t)(merge ? 1 : p->nframes) * p->ntile_tot;
-    const unsigned nbits = bits_for(nkeys + 1);
+    unsigned nbits = bits_for(nkeys + 1);
+    // a tile's entries in the order of their first tap along the slow axis (z,
+    // or y in 2-D), so that a batch of consecutive entries reaches few of the
+    // tile's slow positions and the spread skips the others' products
+    const int sa = p->ndim == 3 ? 0 : 1;
+    int sbits = p->ndim > 1 ? (int)bits_for((uint64_t)p->tile[sa] + p->width[sa] - 1) : 0;
+    if (nbits + sbits > 32) sbits = 0;
+    nbits += sbits;
     DevBuf cnt, off, skeys, svals, skeys2;
     PF_HIP(cnt.alloc(M * 4));
     PF_HIP(off.alloc((M + 1) * 4));
@@ -390,8 +406,8 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
     // item can be read as one piece
     PF_HIP(hipMalloc(&out.slist, (NE + PF_SLIST_PAD) * 4));
     PF_HIP(hipMemsetAsync(out.slist + NE, 0, PF_SLIST_PAD * 4, stream));
-    hipLaunchKernelGGL(k_slist_emit, dim3(nblk(M, TB)), dim3(TB), 0, stream, p->taprec, P, merge,
-                       off.as<uint32_t>(), skeys.as<uint32_t>(), svals.as<int32_t>());
+    hipLaunchKernelGGL(k_slist_emit, dim3(nblk(M, TB)), dim3(TB), 0, stream, p->taprec, P, merge, sa,
+                       sbits, off.as<uint32_t>(), skeys.as<uint32_t>(), svals.as<int32_t>());
     PF_HIP(hipGetLastError());
     size_t rbytes = 0;
     DevBuf rtmp;
@@ -405,7 +421,7 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
     PF_HIP(dend.alloc(nkeys * 4));
     PF_HIP(hipMemsetAsync(dstart.p, 0, nkeys * 4, stream));
     PF_HIP(hipMemsetAsync(dend.p, 0, nkeys * 4, stream));
-    hipLaunchKernelGGL(k_bounds, dim3(nblk(NE, TB)), dim3(TB), 0, stream, skeys2.as<uint32_t>(), NE,
+    hipLaunchKernelGGL(k_bounds, dim3(nblk(NE, TB)), dim3(TB), 0, stream, skeys2.as<uint32_t>(), NE, sbits,
                        dstart.as<int32_t>(), dend.as<int32_t>());
     PF_HIP(hipGetLastError());
     std::vector<int32_t> hs(nkeys), he(nkeys);
@@ -413,28 +429,27 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
     PF_HIP(hipMemcpyAsync(he.data(), dend.p, nkeys * 4, hipMemcpyDeviceToHost, stream));
     PF_HIP(hipStreamSynchronize(stream));
 
-    // work items: heavy tiles split into chunks that a reduce pass sums in order
-    // entries per work item: a chunk is summed serially by one wave, so a
-    // tile far heavier than the rest (the k-space centre of radial and
-    // spiral trajectories) bounds the kernel unless it is split; splitting
-    // tiles of ordinary weight only adds partial-tile traffic.  Split [0]:
-    // above four times the mean entries of a non-empty tile, within
-    // 128..1024.  Split [1]: also small enough that the list makes at least
-    // ~4096 work items (a 2-D grid has few tiles: one wave per tile would
-    // leave most of the GPU idle), within 64..1024; the launch picks it for
-    // batches whose value chunks do not fill the GPU anyway.  Split [2]: twice
-    // split [1]'s item size, for such batches of several value chunks (a
-    // 64-value 2-D B0 adjoint measured 0.204 -> 0.191 ms with it, while
-    // one-chunk batches measured slower).
-    int CH[3] = {p->max_chunk, p->max_chunk, p->max_chunk};
-    if (p->max_chunk <= 0) {
-        int64_t nonempty = 0;
-        for (uint64_t k = 0; k < nkeys; ++k) nonempty += he[k] > hs[k];
-        const int64_t heavy = 4 * NE / std::max<int64_t>(1, nonempty);
-        const int64_t fill = (NE + 4095) / 4096;
-        CH[0] = (int)std::min<int64_t>(1024, std::max<int64_t>(128, heavy));
-        CH[1] = (int)std::min<int64_t>(1024, std::max<int64_t>(PF_SPREAD_MINCH, std::min(heavy, fill)));
-        CH[2] = std::min(CH[0], 2 * CH[1]);
+    // work items: heavy tiles split into chunks that a reduce pass sums in
+    // order.  A chunk is summed serially by one wave, so a tile far heavier
+    // than the rest (the k-space centre of radial and spiral trajectories)
+    // bounds the kernel unless it is split, while every chunk of a split tile
+    // writes and rereads a partial tile of V values per point.  With t the
+    // serial time per entry and s the traffic time of a partial tile (~ V),
+    // NE / n * s + n * t is least at n ~ sqrt(NE V): the factor is the flat
+    // minimum of sweeps over n = 32 .. 2048 (best n: 2-D 107k entries x 64
+    // values 128-256, 183k x 8 96-192, 321k x 16 192-256, 1.67M x 32 384-512;
+    // 3-D 2.8M x 8 256, 8.8M x 8 512, 17M x 32 1024).  Never below four times
+    // the mean of a non-empty tile (at least 128): splitting ordinary tiles
+    // only adds partial tiles.
+    int CH[PF_NSPLIT];
+    int64_t nonempty = 0;
+    for (uint64_t k = 0; k < nkeys; ++k) nonempty += he[k] > hs[k];
+    for (int m = 0; m < PF_NSPLIT; ++m) {
+        const int64_t heavy = std::max<int64_t>(128, 4 * NE / std::max<int64_t>(1, nonempty));
+        const double n = 0.075 * std::sqrt((double)NE * (8 << m));
+        // in steps of sqrt(2), so that neighbouring classes often share their items
+        const int64_t step = (int64_t)std::lround(64.0 * std::exp2(0.5 * std::floor(2.0 * std::log2(std::max(1.0, n / 64.0)) + 0.5)));
+        CH[m] = p->max_chunk > 0 ? p->max_chunk : (int)std::min<int64_t>(1024, std::min(heavy, step));
     }
     // visit tiles in the sample order's Z-order (when it is used), frame by frame
     std::vector<uint64_t> order(nkeys);
@@ -452,42 +467,48 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
         for (uint64_t f = 0; f < nkeys / p->ntile_tot; ++f)
             for (int64_t t = 0; t < p->ntile_tot; ++t) order[q++] = f * p->ntile_tot + tk[t].second;
     }
-    for (int m = 0; m < 3; ++m) {
+    // every split's items, live items and reduce items, gathered on the host
+    // and copied once
+    std::vector<int4> all;
+    struct Piece {
+        size_t items = 0, live = 0, reduce = 0;  // offsets into `all`
+    } piece[PF_NSPLIT];
+    for (int m = 0; m < PF_NSPLIT; ++m) {
         pf_sitems& S = out.split[m];
         bool shared = false;
         for (int q = 0; q < m && !shared; ++q)
             if (CH[q] == CH[m]) {
-                S = out.split[q];  // same arrays
+                S = out.split[q];
+                piece[m] = piece[q];  // same arrays
                 shared = true;
             }
         if (shared) continue;
-        std::vector<int4> items, ritems;
+        std::vector<int4> ritems;
         int slot = 0;
+        piece[m].items = all.size();
         for (uint64_t k : order) {
             int e0 = hs[k], e1 = he[k];
             int n = e1 - e0;
             if (n <= CH[m]) {
-                items.push_back(make_int4((int)k, e0, e1, -1));
+                all.push_back(make_int4((int)k, e0, e1, -1));
             } else {
                 int nch = (n + CH[m] - 1) / CH[m];
                 ritems.push_back(make_int4((int)k, slot, nch, 0));
                 for (int c = 0; c < nch; ++c) {
                     int a = e0 + (int)((int64_t)n * c / nch);
                     int b = e0 + (int)((int64_t)n * (c + 1) / nch);
-                    items.push_back(make_int4((int)k, a, b, slot++));
+                    all.push_back(make_int4((int)k, a, b, slot++));
                 }
             }
         }
-        S.nsitems = (int)items.size();
+        S.nsitems = (int)(all.size() - piece[m].items);
         S.nritems = (int)ritems.size();
         S.nslots = slot;
-        PF_HIP(hipMalloc(&S.sitems, std::max<size_t>(1, items.size()) * sizeof(int4)));
-        PF_HIP(hipMemcpy(S.sitems, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice));
+        piece[m].live = all.size();
         if (!cmask.empty()) {
             // drop the empty tiles lying wholly in columns no sample covers
-            std::vector<int4> live;
-            live.reserve(items.size());
-            for (const int4& it : items) {
+            for (size_t i = piece[m].items; i < piece[m].live; ++i) {
+                const int4 it = all[i];
                 bool keep = it.z > it.y;
                 if (!keep) {
                     const int64_t t = it.x % p->ntile_tot;
@@ -497,15 +518,20 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
                     for (int y = ty * p->tile[1]; y < y1 && !keep; ++y)
                         for (int x = tx * p->tile[2]; x < x1 && !keep; ++x) keep = cmask[(size_t)y * p->os[2] + x] != 0;
                 }
-                if (keep) live.push_back(it);
+                if (keep) all.push_back(it);
             }
-            S.nlsitems = (int)live.size();
-            PF_HIP(hipMalloc(&S.lsitems, std::max<size_t>(1, live.size()) * sizeof(int4)));
-            PF_HIP(hipMemcpy(S.lsitems, live.data(), live.size() * sizeof(int4), hipMemcpyHostToDevice));
+            S.nlsitems = (int)(all.size() - piece[m].live);
         }
-        PF_HIP(hipMalloc(&S.ritems, std::max<size_t>(1, ritems.size()) * sizeof(int4)));
-        if (!ritems.empty())
-            PF_HIP(hipMemcpy(S.ritems, ritems.data(), ritems.size() * sizeof(int4), hipMemcpyHostToDevice));
+        piece[m].reduce = all.size();
+        all.insert(all.end(), ritems.begin(), ritems.end());
+    }
+    PF_HIP(hipMalloc(&out.items, std::max<size_t>(1, all.size()) * sizeof(int4)));
+    PF_HIP(hipMemcpy(out.items, all.data(), all.size() * sizeof(int4), hipMemcpyHostToDevice));
+    for (int m = 0; m < PF_NSPLIT; ++m) {
+        pf_sitems& S = out.split[m];
+        S.sitems = out.items + piece[m].items;
+        S.lsitems = cmask.empty() ? nullptr : out.items + piece[m].live;
+        S.ritems = out.items + piece[m].reduce;
     }
     return PF_OK;
 }
@@ -742,14 +768,7 @@ void pf_plan_free(pf_plan* p) {
     for (int m = 0; m < (alias ? 1 : 2); ++m) {
         const pf_slist& L = p->sl[m];
         if (L.slist) (void)hipFree(L.slist);
-        for (int k = 0; k < 3; ++k) {
-            bool dup = false;  // arrays shared with an earlier split
-            for (int q = 0; q < k; ++q) dup = dup || L.split[q].sitems == L.split[k].sitems;
-            if (dup) continue;
-            if (L.split[k].sitems) (void)hipFree(L.split[k].sitems);
-            if (L.split[k].ritems) (void)hipFree(L.split[k].ritems);
-            if (L.split[k].lsitems) (void)hipFree(L.split[k].lsitems);
-        }
+        if (L.items) (void)hipFree(L.items);
     }
     if (p->fft) pf_fft_destroy(p->fft);
     if (p->fftk) pf_fftk_destroy(p->fftk);
