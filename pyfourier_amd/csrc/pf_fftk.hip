@@ -14,7 +14,8 @@
 //   the X pass writing the deapodised image (sum over B0 segments with the
 //   conjugate maps) in the user layout.
 //
-// Lines of G = 16 Q points (Q in {5, 6, 7, 8, 9, 10, 12, 14, 15, 16, 18, 20,
+// Lines of any other length run a pruned DFT on the FP32 matrix cores
+// (k_dftcol, k_dftrow, k_dftcartrow below).  Lines of G = 16 Q points (Q in {5, 6, 7, 8, 9, 10, 12, 14, 15, 16, 18, 20,
 // 21, 24, 25, 28, 30, 32, 36, 40}: 80-640) and of G = 8 Q points (Q in {5,
 // 7, 9, 15, 21, 25, 35, 45}: 40-360) run register four-step kernels: each
 // thread holds Q values of a line, takes a small DFT in registers, twiddles,
@@ -1827,6 +1828,374 @@ __global__ void __launch_bounds__(FT, PF_FFT_WPE) k_cartrow(AxisFFT A, int64_t n
     }
 }
 
+// ---------------------------------------------------------------------------
+// Passes for any other line length G <= DFT_GMAX (a prime factor above 7, or
+// 7 outside the register sizes): the pruned DFT as a product on the FP32
+// matrix cores.  With the line's rows folded about the origin,
+// a_k = x_k + x_-k and b_k = x_k - x_-k,
+//
+//     X_m, X_-m = sum_k a_k cos(2 pi k m / G)  -/+  i sum_k b_k sin(2 pi k m / G),
+//
+// so a pass between N image rows and G grid rows takes N / 2 x G / 2 real
+// coefficients (2 N flops per complex output instead of 8 N), rows the pad or
+// crop leaves out are never touched, and every length runs the same kernel.
+// Per 4 folded rows a wave takes 2 x 16 output pairs x 16 lines in 8
+// v_mfma_f32_16x16x4_f32; the coefficients come from the twiddle table in LDS
+// by an index that steps mod G, the folded lines from LDS (stride odd, so
+// neither the row-major nor the line-major fill conflicts).  The lines' values
+// are the first operand: a lane ends with 4 neighbouring lines of one row.
+//
+// What bounds it: 2 N flops per output against the 16 bytes a pass must move:
+// level with the 4.9 TB/s copy rate at N ~ 150, so the dense product costs at
+// most 2-3 times a memory-bound pass at N = 400, where a chirp-z transform
+// would take two FFTs of twice the length through LDS.  Measured, fwd + adj
+// with the gather and spread unchanged, rocFFT with separate pad and crop
+// kernels -> these passes: 3-D 113 x 128 x 138 grid x 6 coils (x and z passes
+// here) 1698 -> 565 us, x and z passes 52-71 us each on ~130 MB; 110 x 192 x
+// 198 x 25 coils 13.7 -> 2.0 ms; 2-D 264 x 234 x 5 coils 109 -> 97 us.  Error
+// against 64 bits (whole operators): 2.3e-7 to 5.2e-7, rocFFT's 2.5e-7 to 7.9e-7.
+// ---------------------------------------------------------------------------
+#ifndef PF_FFT_DFT
+#define PF_FFT_DFT 1
+#endif
+constexpr int DFT_GMAX = 1024;
+typedef float dft_f4 __attribute__((ext_vector_type(4)));
+
+// lines per block: the folded rows (K x 4 CT floats) of two blocks fit a CU up
+// to K = 144 (CT = 32) and K = 290 (CT = 16)
+__host__ __device__ constexpr int dft_k4(int K) { return (K + 3) / 4 * 4; }
+__host__ __device__ constexpr int dft_ld(int CT) { return 4 * CT + 1; }
+static inline int dft_ct(int K) { return K <= 144 ? 32 : 16; }
+static inline size_t dft_lds(int G, int K, int CT) {
+    return (size_t)G * sizeof(float2) + (size_t)dft_k4(K) * dft_ld(CT) * sizeof(float);
+}
+
+// fold one pair of rows of a line into the block's LDS
+template <int CT>
+__device__ __forceinline__ void dft_put(float* s_d, int k, int c, float2 p, float2 q) {
+    float* d = s_d + k * dft_ld(CT) + c;
+    d[0] = p.x + q.x;
+    d[CT] = p.y + q.y;
+    d[2 * CT] = p.x - q.x;
+    d[3 * CT] = p.y - q.y;
+}
+
+// the block's folded lines (K rows, padded with zeros to a multiple of 4)
+// times the coefficients: store(m, c0, pos, neg) receives output pair m < M of
+// the 4 lines c0 .. c0 + 3, pos = X_m and neg = X_-m (FWD, exp(-i)) or the
+// other way round (inverse, exp(+i)).  A wave takes units of MW x 16 pairs x
+// 16 lines; blocks sharing the same lines (blockIdx.y) split the units.
+template <int CT, int MW, class Store>
+__device__ __forceinline__ void dft_product(const float* s_d, const float2* s_tw, int K, int M, int G, Store&& store) {
+    constexpr int LD = dft_ld(CT);
+    constexpr int CBN = CT / 16;
+    const int lane = threadIdx.x & 63;
+    const int r16 = lane & 15, kk = lane >> 4;
+    const int units = (M + 16 * MW - 1) / (16 * MW) * CBN;
+    const int nwave = (int)blockDim.x >> 6;
+    for (int u = ((int)threadIdx.x >> 6) + nwave * (int)blockIdx.y; u < units; u += nwave * (int)gridDim.y) {
+        const int cb = u % CBN;
+        int m[MW], i[MW], t[MW];
+        dft_f4 acc[MW][4];
+#pragma unroll
+        for (int q = 0; q < MW; ++q) {
+            m[q] = (u / CBN * MW + q) * 16 + r16;
+            i[q] = (m[q] * kk) % G;
+            t[q] = (4 * m[q]) % G;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[q][j] = dft_f4{0.f, 0.f, 0.f, 0.f};
+        }
+        const float* d = s_d + kk * LD + cb * 16 + r16;
+        // summed 16 rows at a time and the sums added: the rounding error grows
+        // with sqrt(16 + K / 16) instead of sqrt(K) (K = 200: 2.7 times less)
+        for (int k = 0; k < K; k += 16) {
+            dft_f4 part[MW][4];
+#pragma unroll
+            for (int q = 0; q < MW; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) part[q][j] = dft_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int st = 0; st < 4; ++st, d += 4 * LD) {
+                if (k + 4 * st >= K) break;
+                float2 w[MW];
+#pragma unroll
+                for (int q = 0; q < MW; ++q) {
+                    w[q] = s_tw[i[q]];
+                    i[q] += t[q];
+                    i[q] -= i[q] >= G ? G : 0;
+                }
+                const float ar = d[0], ai = d[CT], br = d[2 * CT], bi = d[3 * CT];
+#pragma unroll
+                for (int q = 0; q < MW; ++q) {
+                    part[q][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, w[q].x, part[q][0], 0, 0, 0);
+                    part[q][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, w[q].x, part[q][1], 0, 0, 0);
+                    part[q][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(br, w[q].y, part[q][2], 0, 0, 0);
+                    part[q][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(bi, w[q].y, part[q][3], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < MW; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[q][j] += part[q][j];
+        }
+#pragma unroll
+        for (int q = 0; q < MW; ++q) {
+            if (m[q] >= M) continue;
+            float2 pos[4], neg[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {  // the table holds -sin: R + i S' = X_m of the forward transform
+                pos[r] = make_float2(acc[q][0][r] - acc[q][3][r], acc[q][1][r] + acc[q][2][r]);
+                neg[r] = make_float2(acc[q][0][r] + acc[q][3][r], acc[q][1][r] - acc[q][2][r]);
+            }
+            store(m[q], cb * 16 + 4 * kk, pos, neg);
+        }
+    }
+}
+
+// Column pass of the view (O, rows, I), CT columns per block.  Image rows are
+// centred (row p holds position p - N / 2), grid rows stored (row n holds n
+// mod G); CART: N = G, both sides centred, with the mask and factor of the
+// Cartesian passes.
+template <bool FWD, int CT, int MW, bool CART>
+__global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftcol(int G, int N, int64_t I, const float2* __restrict__ twg,
+                                                const float2* in, float2* out, ColMask cm, CartEpi e) {
+    extern __shared__ __attribute__((aligned(16))) float2 sh[];
+    float2* s_tw = sh;
+    float* s_d = reinterpret_cast<float*>(sh + G);
+    const int64_t nchunk = (I + CT - 1) / CT;
+    const int64_t blk = pf_xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t o = blk / nchunk;
+    const int64_t i0 = (blk % nchunk) * CT;
+    const int h = N / 2, hp = N - N / 2;  // image positions -h .. hp - 1
+    const int half = G / 2 + 1;           // grid positions 0 .. G / 2, paired with their negatives
+    const int K = FWD ? h + 1 : half, M = FWD ? half : h + 1;
+    const int irows = FWD ? N : G, orows = FWD ? G : N;
+    for (int i = threadIdx.x; i < G; i += blockDim.x) s_tw[i] = twg[i];
+    {
+        const int c = threadIdx.x % CT;
+        const int64_t i = i0 + c;
+        const bool ok = i < I && !cm_dead_col(cm, i);
+        const float2* src = in + o * (int64_t)irows * I + i;
+        auto load = [&](int row) {
+            float2 x = src[(int64_t)row * I];
+            if (CART && !FWD) x = c_scale(x, cmask(e, o, G, row, I, i));
+            return x;
+        };
+#pragma unroll 4
+        for (int k = threadIdx.x / CT; k < dft_k4(K); k += blockDim.x / CT) {
+            float2 p = make_float2(0.f, 0.f), q = p;
+            if (FWD || CART) {
+                // FWD: image position k; CART: stored row k sits at the centred row (k + G / 2) mod G,
+                // which for k <= G / 2 is position k (k = G / 2 of an even G only as -k)
+                if (ok && k < hp) p = load(h + k);
+                if (ok && k >= 1 && k <= h) q = load(h - k);
+            } else {
+                if (ok && k < half) p = load(k);
+                if (ok && k >= 1 && 2 * k < G) q = load(G - k);
+            }
+            dft_put<CT>(s_d, k, c, p, q);
+        }
+    }
+    __syncthreads();
+    float2* dst = out + o * (int64_t)orows * I + i0;
+    const int left = (int)std::min<int64_t>(CT, I - i0);
+    auto put = [&](int row, int c0, const float2* v) {
+        float2* d = dst + (int64_t)row * I + c0;
+        float2 x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            x[r] = v[r];
+            if (CART)
+                x[r] = c_scale(x[r], FWD ? e.factor * (c0 + r < left ? cmask(e, o, G, row, I, i0 + c0 + r) : 0.f) : e.factor);
+        }
+        if (c0 + 4 <= left) {
+            __builtin_memcpy(d, x, 32);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+                if (c0 + r < left) d[r] = x[r];
+        }
+    };
+    dft_product<CT, MW>(s_d, s_tw, K, M, G, [&](int m, int c0, const float2* pos, const float2* neg) {
+        const float2* up = FWD ? pos : neg;  // output position +m
+        const float2* dn = FWD ? neg : pos;  // output position -m
+        if (FWD && !CART) {
+            put(m, c0, up);
+            if (m >= 1 && 2 * m < G) put(G - m, c0, dn);
+        } else {
+            if (m < hp) put(h + m, c0, up);
+            if (m >= 1 && m <= h) put(h - m, c0, dn);
+        }
+    });
+}
+
+// Row pass between image rows (coil-major) and grid rows (row, n, v), CT lines
+// per block: line c = (row yy = c / KC, value kc0 + c % KC).  Forward values
+// run over all segments (v = l K Cv + kc, each with its field map); the
+// inverse takes one segment per launch (v = l0 K Cv + kc) and adds it to the
+// image after the first.
+template <bool FWD, int CT, int MW>
+__global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftrow(Geo g, Batch bt, int G, const float2* __restrict__ twg,
+                                                const float* __restrict__ apod, const float2* __restrict__ in,
+                                                float2* __restrict__ out, int KC, int YG, int nkc, int l0, float factor) {
+    extern __shared__ __attribute__((aligned(16))) float2 sh[];
+    __shared__ int64_t s_img[CT], s_grid[CT];  // the lines' image offset (-1: none) and grid offset
+    __shared__ int64_t s_map[CT];              // field-map offset of the line (-1: none)
+    __shared__ float s_ap[CT];
+    float2* s_tw = sh;
+    float* s_d = reinterpret_cast<float*>(sh + G);
+    const int N = g.N[2];
+    const int KCv = bt.K * bt.Cv;
+    const int VT = FWD ? bt.L * KCv : KCv;
+    const int64_t RC = (int64_t)bt.R * bt.Cv;
+    const int64_t nrows = (int64_t)g.N[0] * g.N[1];
+    const int64_t rows_tot = (int64_t)bt.nfg * bt.Cb * nrows;
+    const int64_t blk = pf_xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t row0 = (blk / nkc) * YG;
+    const int kc0 = (int)(blk % nkc) * KC;
+    const int h = N / 2, hp = N - N / 2, half = G / 2 + 1;
+    const int K = FWD ? h + 1 : half, M = FWD ? half : h + 1;
+    const float* apx = apod + g.N[0] + g.N[1];
+    for (int i = threadIdx.x; i < G; i += blockDim.x) s_tw[i] = twg[i];
+    if (threadIdx.x < CT) {
+        const int c = threadIdx.x, yy = c / KC, v = kc0 + c % KC;
+        const int64_t row = row0 + yy;
+        int64_t im = -1, gr = 0, mp = -1;
+        float ap = 0.f;
+        if (yy < YG && v < VT && row < rows_tot) {
+            const int l = FWD ? v / KCv : l0, kc = FWD ? v % KCv : v;
+            int fg, cb;
+            int64_t zy;
+            x_row_decode(bt, row, nrows, fg, cb, zy);
+            const int k = kc / bt.Cv, cv = kc % bt.Cv;
+            const int z = (int)(zy / g.N[1]), y = (int)(zy % g.N[1]);
+            const int ii = bt.nfg > 1 ? fg : (bt.nimg > 1 ? k : 0);
+            im = ((int64_t)(cb * bt.Cv + cv) * bt.nimg + ii) * g.ntot + zy * N;
+            gr = row * G * RC + l * KCv + kc;
+            if (bt.b0s) mp = (int64_t)l * g.ntot + zy * N;
+            ap = apod[z] * apod[g.N[0] + y];
+        }
+        s_img[c] = im;
+        s_grid[c] = gr;
+        s_map[c] = mp;
+        s_ap[c] = ap;
+    }
+    __syncthreads();
+    if (FWD) {
+        // 32 lanes along the image row, 8 lines at a time
+        const int kl = threadIdx.x & 31;
+        for (int c = threadIdx.x >> 5; c < CT; c += blockDim.x >> 5) {
+            const int64_t im = s_img[c], mp = s_map[c];
+            const float ap = s_ap[c];
+            auto load = [&](int p) {
+                float2 x = c_scale(in[im + p], ap * apx[p]);
+                return mp >= 0 ? c_mul(x, bt.b0s[mp + p]) : x;
+            };
+#pragma unroll 2
+            for (int k = kl; k < dft_k4(K); k += 32) {
+                float2 p = make_float2(0.f, 0.f), q = p;
+                if (im >= 0 && k < hp) p = load(h + k);
+                if (im >= 0 && k >= 1 && k <= h) q = load(h - k);
+                dft_put<CT>(s_d, k, c, p, q);
+            }
+        }
+    } else {
+        // lanes along the values when a grid point holds several of them, else along the row
+        const bool vmaj = KC >= 4;
+        const int total = dft_k4(K) * CT;
+#pragma unroll 2
+        for (int q0 = threadIdx.x; q0 < total; q0 += blockDim.x) {
+            const int c = vmaj ? q0 % CT : q0 / dft_k4(K), k = vmaj ? q0 / CT : q0 % dft_k4(K);
+            const float2* src = in + s_grid[c];
+            float2 p = make_float2(0.f, 0.f), q = p;
+            if (s_img[c] >= 0) {
+                if (k < half) p = src[k * RC];
+                if (k >= 1 && 2 * k < G) q = src[(G - k) * RC];
+            }
+            dft_put<CT>(s_d, k, c, p, q);
+        }
+    }
+    __syncthreads();
+    if (FWD) {
+        const bool quads = KC % 4 == 0;  // a lane's 4 lines are 4 neighbouring values
+        dft_product<CT, MW>(s_d, s_tw, K, M, G, [&](int m, int c0, const float2* pos, const float2* neg) {
+            const bool both = m >= 1 && 2 * m < G;
+            if (quads && s_img[c0 + 3] >= 0) {
+                float2* d = out + s_grid[c0];
+                __builtin_memcpy(d + m * RC, pos, 32);
+                if (both) __builtin_memcpy(d + (G - m) * RC, neg, 32);
+                return;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (s_img[c0 + r] < 0) continue;
+                float2* d = out + s_grid[c0 + r];
+                d[m * RC] = pos[r];
+                if (both) d[(G - m) * RC] = neg[r];
+            }
+        });
+    } else {
+        dft_product<CT, MW>(s_d, s_tw, K, M, G, [&](int m, int c0, const float2* pos, const float2* neg) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int c = c0 + r;
+                const int64_t im = s_img[c], mp = s_map[c];
+                if (im < 0) continue;
+                auto put = [&](int p, float2 x) {
+                    if (mp >= 0) x = c_mulc(x, bt.b0s[mp + p]);
+                    x = c_scale(x, factor * s_ap[c] * apx[p]);
+                    out[im + p] = l0 > 0 ? c_add(out[im + p], x) : x;
+                };
+                if (m < hp) put(h + m, neg[r]);
+                if (m >= 1 && m <= h) put(h - m, pos[r]);
+            }
+        });
+    }
+}
+
+// Cartesian row pass: CT contiguous rows of G points per block, centred both
+// sides, in place
+template <bool FWD, int CT, int MW>
+__global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftcartrow(int G, int64_t nrows, const float2* __restrict__ twg, const float2* in,
+                                                    float2* out, CartEpi e) {
+    extern __shared__ __attribute__((aligned(16))) float2 sh[];
+    float2* s_tw = sh;
+    float* s_d = reinterpret_cast<float*>(sh + G);
+    const int64_t r0 = (int64_t)pf_xcd_remap(blockIdx.x, gridDim.x) * CT;
+    const int h = G / 2, hp = G - G / 2, K = h + 1;
+    for (int i = threadIdx.x; i < G; i += blockDim.x) s_tw[i] = twg[i];
+    const int kl = threadIdx.x & 31;
+    for (int c = threadIdx.x >> 5; c < CT; c += blockDim.x >> 5) {
+        const int64_t row = r0 + c;
+        auto load = [&](int j) {
+            const float2 x = in[row * G + j];
+            return FWD ? x : c_scale(x, cmask(e, row, 1, 0, G, j));
+        };
+#pragma unroll 2
+        for (int k = kl; k < dft_k4(K); k += 32) {
+            float2 p = make_float2(0.f, 0.f), q = p;
+            if (row < nrows && k < hp) p = load(h + k);
+            if (row < nrows && k >= 1 && k <= h) q = load(h - k);
+            dft_put<CT>(s_d, k, c, p, q);
+        }
+    }
+    __syncthreads();
+    dft_product<CT, MW>(s_d, s_tw, K, K, G, [&](int m, int c0, const float2* pos, const float2* neg) {
+        const float2* up = FWD ? pos : neg;
+        const float2* dn = FWD ? neg : pos;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t row = r0 + c0 + r;
+            if (row >= nrows) continue;
+            auto put = [&](int j, float2 x) {
+                out[row * G + j] = c_scale(x, FWD ? e.factor * cmask(e, row, 1, 0, G, j) : e.factor);
+            };
+            if (m < hp) put(h + m, up[r]);
+            if (m >= 1 && m <= h) put(h - m, dn[r]);
+        }
+    });
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -1835,6 +2204,7 @@ __global__ void __launch_bounds__(FT, PF_FFT_WPE) k_cartrow(AxisFFT A, int64_t n
 struct pf_fftk_axis {
     int G = 0, N = 0;
     std::vector<int> rad;
+    bool dense = false;  // the matrix-core DFT passes (no radix set, no register size)
     float2* tw = nullptr;
 };
 
@@ -1865,9 +2235,27 @@ static bool fftk_axis_ok(int G) {
     return factorize(G, rad) || (PF_FFTQ && (colq_supported(G) || colq8_supported(G)));
 }
 
-bool pf_fftk_supported(const pf_plan* p) {
+// a length the matrix-core DFT passes take: its folded lines fit a block's LDS
+static bool dft_axis_ok(int G) {
+    return PF_FFT_DFT && G <= DFT_GMAX && dft_lds(G, G / 2 + 1, dft_ct(G / 2 + 1)) <= 158 * 1024;
+}
+
+bool pf_fftk_radix(const pf_plan* p) {
     for (int a = 3 - p->ndim; a < 3; ++a) {
         if (p->os[a] > GBMAX || !fftk_axis_ok(p->os[a])) return false;
+        if (p->shape[a] > p->os[a]) return false;
+    }
+    return true;
+}
+
+// every axis transforms with the fused passes; where one needs the DFT passes
+// the x axis must fit them too, since its row pass then takes over what the
+// register and Stockham row passes refuse (many field-map segments)
+bool pf_fftk_supported(const pf_plan* p) {
+    if (pf_fftk_radix(p)) return true;
+    if (!dft_axis_ok(p->os[2])) return false;
+    for (int a = 3 - p->ndim; a < 3; ++a) {
+        if (p->os[a] > GBMAX || !(fftk_axis_ok(p->os[a]) || dft_axis_ok(p->os[a]))) return false;
         if (p->shape[a] > p->os[a]) return false;
     }
     return true;
@@ -1881,8 +2269,9 @@ int pf_fftk_init(pf_plan* p) {
         X.G = p->os[a];
         X.N = p->shape[a];
         if (!factorize(X.G, X.rad)) {
-            X.rad.clear();  // register passes only (a factor 7)
-            if (!fftk_axis_ok(X.G)) {
+            X.rad.clear();  // register passes only (a factor 7), or the DFT passes
+            X.dense = !fftk_axis_ok(X.G);
+            if (X.dense && !dft_axis_ok(X.G)) {
                 pf_fftk_destroy(f);
                 return pf_fail(PF_ERR_UNSUPPORTED, "grid size has prime factors other than 2, 3, 5");
             }
@@ -1907,6 +2296,38 @@ int pf_fftk_init(pf_plan* p) {
             if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) {
                 pf_fftk_destroy(f);
                 return pf_fail(PF_ERR_HIP, "could not raise the FFT kernels' LDS limit");
+            }
+    }
+    if (!pf_fftk_radix(p)) {
+        const void* kernels[] = {
+            reinterpret_cast<const void*>(k_dftcol<true, 32, 2, false>),
+            reinterpret_cast<const void*>(k_dftcol<true, 32, 2, true>),
+            reinterpret_cast<const void*>(k_dftrow<true, 32, 2>),
+            reinterpret_cast<const void*>(k_dftcartrow<true, 32, 2>),
+            reinterpret_cast<const void*>(k_dftcol<false, 32, 2, false>),
+            reinterpret_cast<const void*>(k_dftcol<false, 32, 2, true>),
+            reinterpret_cast<const void*>(k_dftrow<false, 32, 2>),
+            reinterpret_cast<const void*>(k_dftcartrow<false, 32, 2>),
+            reinterpret_cast<const void*>(k_dftcol<true, 16, 2, false>),
+            reinterpret_cast<const void*>(k_dftcol<true, 16, 2, true>),
+            reinterpret_cast<const void*>(k_dftrow<true, 16, 2>),
+            reinterpret_cast<const void*>(k_dftcartrow<true, 16, 2>),
+            reinterpret_cast<const void*>(k_dftcol<false, 16, 2, false>),
+            reinterpret_cast<const void*>(k_dftcol<false, 16, 2, true>),
+            reinterpret_cast<const void*>(k_dftrow<false, 16, 2>),
+            reinterpret_cast<const void*>(k_dftcartrow<false, 16, 2>),
+            reinterpret_cast<const void*>(k_dftcol<true, 16, 1, false>),
+            reinterpret_cast<const void*>(k_dftcol<true, 16, 1, true>),
+            reinterpret_cast<const void*>(k_dftrow<true, 16, 1>),
+            reinterpret_cast<const void*>(k_dftcartrow<true, 16, 1>),
+            reinterpret_cast<const void*>(k_dftcol<false, 16, 1, false>),
+            reinterpret_cast<const void*>(k_dftcol<false, 16, 1, true>),
+            reinterpret_cast<const void*>(k_dftrow<false, 16, 1>),
+            reinterpret_cast<const void*>(k_dftcartrow<false, 16, 1>)};
+        for (const void* k : kernels)
+            if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024) != hipSuccess) {
+                pf_fftk_destroy(f);
+                return pf_fail(PF_ERR_HIP, "could not raise the DFT kernels' LDS limit");
             }
     }
     p->fftk = f;
@@ -1973,10 +2394,136 @@ size_t pf_fftk_extra_bytes(const pf_plan* p, const pf_batch& b) {
     return 0;
 }
 
+// Shape of a DFT pass over `lines` lines in groups of 32 or 16 per block (each
+// group size gives its number of blocks): 32 lines and 32 output pairs per
+// wave step when that alone gives every CU two blocks; with fewer lines 16 of
+// each, and the blocks of a group repeated so that they split its outputs
+// (each refolds the lines), or, in place, where one block's stores would meet
+// another's loads, up to 16 waves per block.  2-D 264 x 234 grid x 5 coils (37
+// + 33 blocks of 32 lines), fwd + adj 148 us with whole groups, 97 us split.
+struct DftShape {
+    int K, CT, MW, threads;
+    dim3 grid;
+    size_t lds;
+};
+
+template <class Blocks>
+static int dft_shape(const pf_fftk_axis& X, bool fwd, bool split, Blocks&& blocks, DftShape& d) {
+    const int h = X.N / 2 + 1, half = X.G / 2 + 1;
+    d.K = fwd ? h : half;
+    const int M = fwd ? half : h;
+    d.CT = dft_ct(d.K);
+    d.MW = 2;
+    d.threads = 256;
+    int64_t nblk = blocks(d.CT), parts = 1;
+    if (nblk < 512) {
+        d.CT = 16;
+        d.MW = 1;
+        nblk = blocks(16);
+        const int rounds = ((M + 15) / 16 + 3) / 4;  // of 4 waves over the output units
+        if (split)
+            parts = std::max<int64_t>(1, std::min<int64_t>(rounds, 512 / std::max<int64_t>(1, nblk)));
+        else
+            d.threads = 256 * std::min(4, rounds);
+    }
+    if (nblk > 0x7fffffff) return pf_fail(PF_ERR_UNSUPPORTED, "too many FFT lines");
+    d.grid = dim3((unsigned)nblk, (unsigned)parts);
+    d.lds = dft_lds(X.G, d.K, d.CT);
+    return PF_OK;
+}
+
+static int launch_dft_col(const pf_fftk_axis& X, bool fwd, bool cart, int64_t O, int64_t I, const float2* src,
+                          float2* dst, const ColMask& cm, const CartEpi& e, hipStream_t s) {
+    DftShape d;
+    const int rc = dft_shape(X, fwd, src != dst, [&](int CT) { return O * ((I + CT - 1) / CT); }, d);
+    if (rc != PF_OK || d.grid.x < 1) return rc;
+#define PF_DFTCOL(F, T, W, C) \
+    hipLaunchKernelGGL((k_dftcol<F, T, W, C>), d.grid, dim3(d.threads), d.lds, s, X.G, X.N, I, X.tw, src, dst, cm, e)
+#define PF_DFTCOL2(F, C)                          \
+    if (d.CT == 32) PF_DFTCOL(F, 32, 2, C);       \
+    else if (d.MW == 2) PF_DFTCOL(F, 16, 2, C);   \
+    else PF_DFTCOL(F, 16, 1, C)
+    if (cart && fwd) {
+        PF_DFTCOL2(true, true);
+    } else if (cart) {
+        PF_DFTCOL2(false, true);
+    } else if (fwd) {
+        PF_DFTCOL2(true, false);
+    } else {
+        PF_DFTCOL2(false, false);
+    }
+#undef PF_DFTCOL2
+#undef PF_DFTCOL
+    PF_HIP(hipGetLastError());
+    return PF_OK;
+}
+
+static int launch_dft_row(const pf_plan* p, const pf_batch& b, bool fwd, const float2* src, float2* dst, float factor,
+                          hipStream_t s) {
+    const pf_fftk_axis& X = p->fftk->ax[2];
+    const int KCv = b.K * b.Cv, VT = fwd ? b.L * KCv : KCv;
+    const int64_t rows = (int64_t)b.nfg * b.Cb * p->shape[0] * p->shape[1];
+    int KC = 1, YG = 1, nkc = 1;
+    DftShape d;
+    const int rc = dft_shape(
+        X, fwd, true,
+        [&](int CT) {
+            KC = std::min(VT, CT);
+            YG = CT / KC;
+            nkc = (VT + KC - 1) / KC;
+            return (rows + YG - 1) / YG * nkc;
+        },
+        d);
+    if (rc != PF_OK || d.grid.x < 1) return rc;
+    const Geo g = geo_of(p);
+    const Batch t = batch_of(b);
+#define PF_DFTROW(F, T, W, L0, FAC)                                                                                  \
+    hipLaunchKernelGGL((k_dftrow<F, T, W>), d.grid, dim3(d.threads), d.lds, s, g, t, X.G, X.tw, p->apod, src, dst, KC, YG, \
+                       nkc, L0, FAC)
+#define PF_DFTROW2(F, L0, FAC)                          \
+    if (d.CT == 32) PF_DFTROW(F, 32, 2, L0, FAC);       \
+    else if (d.MW == 2) PF_DFTROW(F, 16, 2, L0, FAC);   \
+    else PF_DFTROW(F, 16, 1, L0, FAC)
+    if (fwd) {
+        PF_DFTROW2(true, 0, 1.0f);
+    } else {
+        for (int l = 0; l < b.L; ++l) {  // the segments' images are summed in launch order
+            PF_DFTROW2(false, l, factor);
+        }
+    }
+#undef PF_DFTROW2
+#undef PF_DFTROW
+    PF_HIP(hipGetLastError());
+    return PF_OK;
+}
+
+static int launch_dft_cartrow(const pf_fftk_axis& X, bool fwd, int64_t nrows, const float2* src, float2* dst,
+                              const CartEpi& e, hipStream_t s) {
+    DftShape d;
+    const int rc = dft_shape(X, fwd, src != dst, [&](int CT) { return (nrows + CT - 1) / CT; }, d);
+    if (rc != PF_OK || d.grid.x < 1) return rc;
+#define PF_DFTCROW(F, T, W) \
+    hipLaunchKernelGGL((k_dftcartrow<F, T, W>), d.grid, dim3(d.threads), d.lds, s, X.G, nrows, X.tw, src, dst, e)
+#define PF_DFTCROW2(F)                       \
+    if (d.CT == 32) PF_DFTCROW(F, 32, 2);    \
+    else if (d.MW == 2) PF_DFTCROW(F, 16, 2); \
+    else PF_DFTCROW(F, 16, 1)
+    if (fwd) {
+        PF_DFTCROW2(true);
+    } else {
+        PF_DFTCROW2(false);
+    }
+#undef PF_DFTCROW2
+#undef PF_DFTCROW
+    PF_HIP(hipGetLastError());
+    return PF_OK;
+}
+
 static int launch_x(const pf_plan* p, const pf_batch& b, bool fwd, const float2* src, float2* dst, float factor,
                     hipStream_t s) {
     const pf_fftk_axis& X = p->fftk->ax[2];
     const int KCv = b.K * b.Cv;
+    if (X.dense) return launch_dft_row(p, b, fwd, src, dst, factor, s);
     if (X.G == 256 && b.L == 1 && !b.b0s) {
         const int BX = fwd ? X256_BF : X256_BA;
         const int KC = std::min(KCv, BX);
@@ -2129,9 +2676,13 @@ static int launch_x(const pf_plan* p, const pf_batch& b, bool fwd, const float2*
         PF_HIP(hipGetLastError());
         return PF_OK;
     }
-    if (X.rad.empty())
+    const bool radix = pf_fftk_radix(p);
+    if (X.rad.empty()) {
+        if (!radix) return launch_dft_row(p, b, fwd, src, dst, factor, s);
         return pf_fail(PF_ERR_UNSUPPORTED, kNoStockham);
+    }
     AxisFFT A = axis_desc(X);
+    if ((int64_t)b.L * X.G > GBMAX && !radix) return launch_dft_row(p, b, fwd, src, dst, factor, s);
     if ((int64_t)b.L * X.G > GBMAX)
         return pf_fail(PF_ERR_UNSUPPORTED, "too many B0 segments for the fused FFT at this grid size");
     XBlk xb;
@@ -2160,6 +2711,7 @@ static int launch_x(const pf_plan* p, const pf_batch& b, bool fwd, const float2*
 static int launch_col(const pf_plan* p, int axis, bool fwd, int64_t O, int64_t I, const float2* src, float2* dst,
                       hipStream_t s, ColMask cm = ColMask{nullptr, 0, 1}) {
     const pf_fftk_axis& X = p->fftk->ax[axis];
+    if (X.dense) return launch_dft_col(X, fwd, false, O, I, src, dst, cm, CartEpi{nullptr, 1, 0, 1.0f}, s);
     if (X.G == 512 && PF_FFT512) {
         const bool wide = O * I >= C512_MIN;
         const int B = wide ? C512_B : C512_BS;
@@ -2286,7 +2838,8 @@ static int launch_col(const pf_plan* p, int axis, bool fwd, int64_t O, int64_t I
 bool pf_fftk_masked(const pf_plan* p) {
     if (!PF_COLMASK || p->ndim != 3 || !p->colmask || !p->fftk) return false;
     const int G = p->fftk->ax[0].G;
-    return G == 256 || (G == 512 && PF_FFT512) || (PF_FFTQ && (colq_supported(G) || colq8_supported(G)));
+    return p->fftk->ax[0].dense || G == 256 || (G == 512 && PF_FFT512) ||
+           (PF_FFTQ && (colq_supported(G) || colq8_supported(G)));
 }
 
 // image -> grid (deapodise, pad, FFT); `extra` holds pf_fftk_extra_bytes
@@ -2335,6 +2888,7 @@ int pf_fftk_adjoint(pf_plan* p, const pf_batch& b, float2* grid, float2* img, fl
 static int cart_col(const pf_plan* p, int axis, bool fwd, int64_t O, int64_t I, const float2* src, float2* dst,
                     const CartEpi& e, hipStream_t s) {
     const pf_fftk_axis& X = p->fftk->ax[axis];
+    if (X.dense) return launch_dft_col(X, fwd, true, O, I, src, dst, ColMask{nullptr, 0, 1}, e, s);
     if (X.G == 256) {
         const int B = fwd ? CC256_BF : CC256_BA;
         const int64_t nblk = O * ((I + B - 1) / B);
@@ -2450,6 +3004,7 @@ static int cart_col(const pf_plan* p, int axis, bool fwd, int64_t O, int64_t I, 
 static int cart_row(const pf_plan* p, bool fwd, int64_t nrows, const float2* src, float2* dst, const CartEpi& e,
                     hipStream_t s) {
     const pf_fftk_axis& X = p->fftk->ax[2];
+    if (X.dense) return launch_dft_cartrow(X, fwd, nrows, src, dst, e, s);
     if (X.G == 256) {
         const int64_t nblk = (nrows + 15) / 16;
         if (nblk > 0x7fffffff) return pf_fail(PF_ERR_UNSUPPORTED, "too many FFT rows");

@@ -219,6 +219,7 @@ int pf_noalloc_prepare();  // this device's pf_nufft_noalloc scratch address, at
 
 // fused deapodise/pad/FFT and inverse FFT/crop/deapodise (pf_fftk.hip)
 bool pf_fftk_supported(const pf_plan* p);
+bool pf_fftk_radix(const pf_plan* p);  // by the radix and register passes alone
 int pf_fftk_init(pf_plan* p);
 int pf_fftk_ready(const pf_plan* p);  // PF_OK when pf_fftk_init has run
 void pf_fftk_destroy(struct pf_fftk* f);

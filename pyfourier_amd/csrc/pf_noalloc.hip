@@ -51,9 +51,9 @@ extern "C" int pf_nufft_noalloc(pf_plan* p, const pf_batch_desc* d, int op, cons
                                 const float* weight, int norm, void* stream) {
     if (!p) return pf_fail(PF_ERR_ARG, "null plan");
     if (op != 0 && op != 1) return pf_fail(PF_ERR_ARG, "op must be 0 (forward) or 1 (adjoint)");
-    if (!pf_fftk_supported(p))
+    if (!pf_fftk_radix(p))
         return pf_fail(PF_ERR_UNSUPPORTED,
-                       "pf_nufft_noalloc needs grid sizes 2^a 3^b 5^c (other sizes run rocFFT, which allocates)");
+                       "pf_nufft_noalloc needs grid sizes 2^a 3^b 5^c");
     int dev = -1;
     PF_HIP(hipGetDevice(&dev));
     if (dev != p->device) return pf_fail(PF_ERR_ARG, "the plan lives on another device than the current one");
