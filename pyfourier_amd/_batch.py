@@ -96,14 +96,13 @@ class _Group:
         L = _lib.lib()
         desc = _lib.BatchDesc()
         desc.batch, desc.nseg, desc.ncoeff, desc.nt = self.nbatch, 1, 0, 1
-        nbytes = ctypes.c_size_t()
-        _lib.check(L.pf_workspace_size(self.native.handle, ctypes.byref(desc), int(adjoint), ctypes.byref(nbytes)))
-        ws = torch.empty(max(1, nbytes.value), dtype=torch.uint8, device=self.device)
+        nbytes = self.native.workspace_bytes(desc, int(adjoint))
+        ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=self.device)
         fn = L.pf_nufft_adj if adjoint else L.pf_nufft
         src, dst = (self.kspace, self.images) if adjoint else (self.images, self.kspace)
-        with torch.cuda.device(self.device):
+        with _lib.on(self.device):
             _lib.check(fn(self.native.handle, ctypes.byref(desc), _lib.ptr(src), _lib.ptr(dst),
-                          _lib.ptr(self.weight), code, _lib.ptr(ws), nbytes.value, _lib.stream_of(self.device)))
+                          _lib.ptr(self.weight), code, _lib.ptr(ws), nbytes, _lib.stream_of(self.device)))
 
 
 class NUFFTBatch:
@@ -184,13 +183,13 @@ class NUFFTBatch:
 
     def _replay(self, adjoint: bool, code: int):
         if not self.use_graph:
-            with torch.cuda.device(self.device):
+            with _lib.on(self.device):
                 self._launch(adjoint, code)
             return
         key = (adjoint, code)
         g = self._graphs.get(key)
         if g is None:
-            with torch.cuda.device(self.device):
+            with _lib.on(self.device):
                 # warm-up outside the capture: lazily built FFT state and
                 # the caching allocator's blocks exist before recording
                 side = torch.cuda.Stream(self.device)

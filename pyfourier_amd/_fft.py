@@ -25,6 +25,7 @@ undefined variable).
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -200,7 +201,7 @@ class _CartCall:
             n = ctypes.c_size_t()
             _lib.check(L.pf_cart_workspace_size(self.native.handle, ctypes.byref(desc), self.T, ctypes.byref(n)))
             ws = torch.empty(max(1, n.value), dtype=torch.uint8, device=self.dev)
-            with torch.cuda.device(self.dev):
+            with _lib.on(self.dev):
                 _lib.check(fn(self.native.handle, ctypes.byref(desc), self.T, _lib.ptr(x), _lib.ptr(dst), int(code),
                               _lib.ptr(ws), n.value, stream))
             if i:
@@ -255,7 +256,7 @@ def _apply(ndim, data, mask, plan, basis, zmap, L, nbins, dt, T, L_batch_size, n
     plan.to(dev)
     dtype = x.dtype
     batch, nfr, planes, has_axis = _layout(x, ndim, plan, basis, inverse)
-    C = int(np.prod(batch)) if batch else 1
+    C = math.prod(batch)
     call = _CartCall(plan, dev, basis, nfr)
     xin = x.to(device=dev, dtype=torch.complex64).reshape((C, planes) + tuple(plan.shape)).contiguous()
     y = _CartFn.apply(xin, call, inverse, code)
@@ -325,7 +326,7 @@ def _fft_util(data, axes, norm, centered, inverse):
     if not centered:
         xm = torch.fft.fftshift(xm, dim=sax)
     bshape = tuple(xm.shape[:-d])
-    C = int(np.prod(bshape)) if bshape else 1
+    C = math.prod(bshape)
     call = _CartCall(_util_plan(shape, dev), dev, None, 1)
     code = _UTIL_CODES[norm][1 if inverse else 0]
     y = _CartFn.apply(xm.reshape((C, 1) + shape).contiguous(), call, inverse, code).reshape(bshape + shape)

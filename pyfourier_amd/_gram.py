@@ -28,6 +28,7 @@ accepts 1-, 2- or 3-D grids (the reference asserts 2-D).
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -169,7 +170,7 @@ def _apply(x: torch.Tensor, gm: GramMatrix) -> torch.Tensor:
     _lib.check(L.pf_toeplitz_workspace_size(h, int(C), ctypes.byref(n)))
     ws = torch.empty(max(1, n.value), dtype=torch.uint8, device=x.device)
     zs = None if gm.zmap_s_kernel is None else gm.zmap_s_kernel.reshape(gm.nseg, -1).contiguous()
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.check(L.pf_toeplitz_apply(h, int(C), _lib.ptr(x), _lib.ptr(out), _lib.ptr(zs), _lib.ptr(ws), n.value,
                                        _lib.stream_of(x.device)))
     return out
@@ -210,7 +211,7 @@ def gram(image, gram_matrix: GramMatrix, norm=None, device="cpu"):
         batch = tuple(x.shape[: -(d + 1)])
     else:
         batch = tuple(x.shape[:-d])
-    C = int(np.prod(batch)) if batch else 1
+    C = math.prod(batch)
     dtype = x.dtype
     xin = x.to(device=dev, dtype=torch.complex64).reshape((C, planes) + shp).contiguous()
     y = _GramFn.apply(xin, gm).reshape(x.shape)

@@ -7,6 +7,7 @@ is missing the import of an operator fails with a clear error.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -148,8 +149,20 @@ def check(rc: int) -> None:
 
 
 def ptr(t: "torch.Tensor | None"):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_HERE_ALREADY = contextlib.nullcontext()
 
 
 def stream_of(device: "torch.device"):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """Handle of the device's current stream."""
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
+
+
+def on(device: "torch.device"):
+    """Context in which `device` is current; nothing to enter where it already is."""
+    return _HERE_ALREADY if torch.cuda.current_device() == device.index else torch.cuda.device(device)

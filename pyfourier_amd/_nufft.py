@@ -97,8 +97,10 @@ class _Call:
         self.weight_full = None  # anything else, applied with torch
         if weight is not None:
             w = _to_torch(weight).to(device)
-            if not torch.is_complex(w):
-                ks = (self.interp.nframes,) + tuple(self.interp.dshape)
+            ks = (self.interp.nframes,) + tuple(self.interp.dshape)
+            if w.dtype is torch.float32 and w.shape == ks and w.is_contiguous():
+                self.weight_flat = w.reshape(-1)
+            elif not torch.is_complex(w):
                 try:
                     we = torch.broadcast_to(w.to(torch.float32), ks)
                     if we.dim() >= w.dim():
@@ -159,18 +161,17 @@ class _Call:
         acc = None
         for seg in self.segments:
             desc = self.desc(C, seg)
-            nbytes = ctypes.c_size_t()
-            _lib.check(L.pf_workspace_size(self.native.handle, ctypes.byref(desc), 0, ctypes.byref(nbytes)))
-            ws = torch.empty(max(1, nbytes.value), dtype=torch.uint8, device=self.device)
+            nbytes = self.native.workspace_bytes(desc, 0)
+            ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=self.device)
             y = out if acc is None else torch.empty_like(out)
-            with torch.cuda.device(self.device):
+            with _lib.on(self.device):
                 if stage_timer.active is not None:
                     self._staged_forward(desc, x, y, ws, norm_code)
                 else:
                     _lib.check(
                         L.pf_nufft(
                             self.native.handle, ctypes.byref(desc), _lib.ptr(x), _lib.ptr(y),
-                            _lib.ptr(self.weight_flat), norm_code, _lib.ptr(ws), nbytes.value,
+                            _lib.ptr(self.weight_flat), norm_code, _lib.ptr(ws), nbytes,
                             _lib.stream_of(self.device),
                         )
                     )
@@ -190,13 +191,12 @@ class _Call:
         fac = self._factor(norm_code, False)
         for seg in self.segments:
             desc = self.desc(C, seg)
-            nbytes = ctypes.c_size_t()
-            _lib.check(L.pf_workspace_size(self.native.handle, ctypes.byref(desc), 1, ctypes.byref(nbytes)))
-            ws = torch.empty(max(1, nbytes.value), dtype=torch.uint8, device=self.device)
+            nbytes = self.native.workspace_bytes(desc, 1)
+            ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=self.device)
             grid, ys, fws, _ = self._split_ws(desc, ws)
             y = out if acc is None else torch.empty_like(out)
             h, d, st = self.native.handle, ctypes.byref(desc), _lib.stream_of(self.device)
-            with torch.cuda.device(self.device):
+            with _lib.on(self.device):
                 _lib.check(L.pf_pad_fft(h, d, _lib.ptr(x), _lib.ptr(grid), _lib.ptr(fws), st))
                 _lib.check(L.pf_interp(h, d, _lib.ptr(grid), _lib.ptr(ys), st))
                 _lib.check(L.pf_unsort_samples(h, d, _lib.ptr(ys), _lib.ptr(y), _lib.ptr(self.weight_flat), fac, st))
@@ -230,12 +230,10 @@ class _Call:
             if kept is not None:
                 ws = kept[i]
             else:
-                nbytes = ctypes.c_size_t()
-                _lib.check(L.pf_workspace_size(self.native.handle, ctypes.byref(desc), 1, ctypes.byref(nbytes)))
-                ws = torch.empty(max(1, nbytes.value), dtype=torch.uint8, device=self.device)
+                ws = torch.empty(max(1, self.native.workspace_bytes(desc, 1)), dtype=torch.uint8, device=self.device)
             grid, ys, fws, _ = self._split_ws(desc, ws)
             h_, d, st = self.native.handle, ctypes.byref(desc), _lib.stream_of(self.device)
-            with torch.cuda.device(self.device):
+            with _lib.on(self.device):
                 if kept is None:
                     _lib.check(L.pf_pad_fft(h_, d, _lib.ptr(img), _lib.ptr(grid), _lib.ptr(fws), st))
                 _lib.check(L.pf_sort_samples(h_, d, _lib.ptr(h), _lib.ptr(ys), _lib.ptr(self.weight_flat), st))
@@ -244,7 +242,7 @@ class _Call:
 
     # ---- stage-by-stage execution (timing) ---------------------------------
     def _factor(self, norm_code: int, adjoint: bool) -> float:
-        g = float(np.prod(self.interp.os_shape))
+        g = float(math.prod(self.interp.os_shape))
         f = 1.0 / self.native.info.scale
         if norm_code == _lib.PF_NORM_ORTHO:
             return f / math.sqrt(g)
@@ -297,18 +295,17 @@ class _Call:
         acc = None
         for seg in self.segments:
             desc = self.desc(C, seg)
-            nbytes = ctypes.c_size_t()
-            _lib.check(L.pf_workspace_size(self.native.handle, ctypes.byref(desc), 1, ctypes.byref(nbytes)))
-            ws = torch.empty(max(1, nbytes.value), dtype=torch.uint8, device=self.device)
+            nbytes = self.native.workspace_bytes(desc, 1)
+            ws = torch.empty(max(1, nbytes), dtype=torch.uint8, device=self.device)
             x = out if acc is None else torch.empty_like(out)
-            with torch.cuda.device(self.device):
+            with _lib.on(self.device):
                 if stage_timer.active is not None:
                     self._staged_adjoint(desc, y, x, ws, norm_code)
                 else:
                     _lib.check(
                         L.pf_nufft_adj(
                             self.native.handle, ctypes.byref(desc), _lib.ptr(y), _lib.ptr(x),
-                            _lib.ptr(self.weight_flat), norm_code, _lib.ptr(ws), nbytes.value,
+                            _lib.ptr(self.weight_flat), norm_code, _lib.ptr(ws), nbytes,
                             _lib.stream_of(self.device),
                         )
                     )
@@ -331,7 +328,7 @@ def _image_layout(image: torch.Tensor, call: _Call):
     else:
         nimg = 1
         batch_shape = tuple(image.shape[:-d])
-    C = int(np.prod(batch_shape)) if batch_shape else 1
+    C = math.prod(batch_shape)
     return batch_shape, C, nimg
 
 
@@ -346,7 +343,7 @@ def _kspace_layout(kspace: torch.Tensor, call: _Call):
         batch_shape = tuple(kspace.shape[: -(nd + 1)])
     else:
         batch_shape = tuple(kspace.shape[:-nd])
-    C = int(np.prod(batch_shape)) if batch_shape else 1
+    C = math.prod(batch_shape)
     return batch_shape, C
 
 
@@ -442,10 +439,11 @@ class _NUFFTAdjTrajFn(torch.autograd.Function):
 def _restore(out: torch.Tensor, dtype, backend_numpy: bool, idevice):
     if not dtype.is_complex:
         out = out.real
-    out = out.to(dtype)
+    if out.dtype is not dtype:
+        out = out.to(dtype)
     if backend_numpy:
         return out.detach().cpu().numpy()
-    return out.to(idevice)
+    return out if out.device == idevice else out.to(idevice)
 
 
 def _traj_tensor(coord, call):

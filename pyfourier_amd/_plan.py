@@ -83,6 +83,18 @@ class NativePlan:
         self.info = info
         self._lib = L
         self._perm = None
+        self._ws = {}  # workspace bytes by (batch, ncoeff, nseg, field map, op): sizes only
+
+    def workspace_bytes(self, desc, op: int) -> int:
+        """pf_workspace_size of a call; it depends on the batch description's
+        counts and on which of its arrays are given, not on their contents."""
+        key = (desc.batch, desc.ncoeff, desc.nseg, desc.b0_temporal is not None, desc.basis is not None, op)
+        n = self._ws.get(key)
+        if n is None:
+            size = ctypes.c_size_t()
+            _lib.check(self._lib.pf_workspace_size(self.handle, ctypes.byref(desc), op, ctypes.byref(size)))
+            n = self._ws[key] = size.value
+        return n
 
     def permutation(self) -> torch.Tensor:
         """Original sample index (frame * npts + j) of every tile-sorted position."""
@@ -130,7 +142,7 @@ class Interpolator:
 
     @property
     def npts(self) -> int:
-        return int(np.prod(self.dshape))
+        return math.prod(self.dshape)
 
     def native(self, device: torch.device) -> NativePlan:
         key = (device.type, device.index)
