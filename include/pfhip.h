@@ -410,6 +410,15 @@ int pf_voronoi_area_2d(const double* pts, const int* bucket_start, int nx, int n
                        long long npoints, const unsigned char* open, const int* list, long long nlist, void* work,
                        int work_vertices, double* area, int* status, void* stream);
 
+/* ---- batches of arrays ------------------------------------------------ */
+
+/* Copies n arrays of rows[i] x len[i] complex64 values, contiguous at src[i],
+ * to dst[i] with dst_stride[i] values between rows (the items of an uneven
+ * batch into its static buffers; no reference counterpart).  The pointer and
+ * size arrays are host memory, read before the call returns. */
+int pf_copy_items(int n, const void* const* src, void* const* dst, const long long* rows, const long long* len,
+                  const long long* dst_stride, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

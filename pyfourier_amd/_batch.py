@@ -230,7 +230,21 @@ class NUFFTBatch:
             if s.numel() != d.numel():
                 raise ValueError(f"item of {s.numel()} values does not fit a buffer of shape {tuple(d.shape)}")
             srcs.append(s.reshape(d.shape).to(device=self.device, dtype=torch.complex64))
-        torch._foreach_copy_(dst, srcs)
+        if torch.is_grad_enabled() and any(s.requires_grad for s in srcs):
+            torch._foreach_copy_(dst, srcs)
+            return
+        # one native launch for all items: the buffers are (nbatch, planes or
+        # frames, ...) views whose rows (everything behind the batch axis) are
+        # contiguous
+        srcs = [s.resolve_conj().resolve_neg().contiguous() for s in srcs]
+        n = len(dst)
+        rows = [int(d.shape[0]) for d in dst]
+        LL = ctypes.c_longlong * n
+        with _lib.on(self.device):
+            _lib.check(_lib.lib().pf_copy_items(
+                n, (ctypes.c_void_p * n)(*[_lib.ptr(s) for s in srcs]), (ctypes.c_void_p * n)(*[_lib.ptr(d) for d in dst]),
+                LL(*rows), LL(*[d.numel() // max(1, r) for d, r in zip(dst, rows)]), LL(*[int(d.stride(0)) for d in dst]),
+                _lib.stream_of(self.device)))
 
 
 def plan_nufft_batch(coords, shapes, nbatch=1, width=4, oversamp=1.25, weights=None, basis=None, norm=None,

@@ -117,6 +117,7 @@ _SIG = {
     "pf_unsort_samples": (_I, [_VP, ctypes.POINTER(BatchDesc), _VP, _VP, _VP, ctypes.c_float, _VP]),
     "pf_voronoi_area_2d": (_I, [_VP, _VP, _I, _I, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_longlong,
                                 _VP, _VP, ctypes.c_longlong, _VP, _I, _VP, _VP, _VP]),
+    "pf_copy_items": (_I, [_I, ctypes.POINTER(_VP), ctypes.POINTER(_VP)] + [ctypes.POINTER(ctypes.c_longlong)] * 3 + [_VP]),
 }
 
 EXPORTED = tuple(_SIG)
