@@ -1882,7 +1882,8 @@ __device__ __forceinline__ void dft_put(float* s_d, int k, int c, float2 p, floa
 
 // the block's folded lines (K rows, padded with zeros to a multiple of 4)
 // times the coefficients: store(m, c0, pos, neg) receives output pair m < M of
-// the 4 lines c0 .. c0 + 3, pos = X_m and neg = X_-m (FWD, exp(-i)) or the
+// the lines c0, c0 + 1, c0 + 8 and c0 + 9 (so that the 4 lanes of a row write 64
+// contiguous bytes per store where lines are neighbours), pos = X_m and neg = X_-m (FWD, exp(-i)) or the
 // other way round (inverse, exp(+i)).  A wave takes units of MW x 16 pairs x
 // 16 lines; blocks sharing the same lines (blockIdx.y) split the units.
 template <int CT, int MW, class Store>
@@ -1905,38 +1906,52 @@ __device__ __forceinline__ void dft_product(const float* s_d, const float2* s_tw
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[q][j] = dft_f4{0.f, 0.f, 0.f, 0.f};
         }
-        const float* d = s_d + kk * LD + cb * 16 + r16;
+        // operand row 4 q + r holds line 8 (r / 2) + 2 q + r % 2
+        const float* d = s_d + kk * LD + cb * 16 + (r16 & 2) * 4 + (r16 >> 2) * 2 + (r16 & 1);
         // summed 16 rows at a time and the sums added: the rounding error grows
         // with sqrt(16 + K / 16) instead of sqrt(K) (K = 200: 2.7 times less)
-        for (int k = 0; k < K; k += 16) {
-            dft_f4 part[MW][4];
+        dft_f4 part[MW][4];
+        auto clear = [&]() {
 #pragma unroll
             for (int q = 0; q < MW; ++q)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) part[q][j] = dft_f4{0.f, 0.f, 0.f, 0.f};
+        };
+        auto step = [&]() {  // 4 rows
+            float2 w[MW];
 #pragma unroll
-            for (int st = 0; st < 4; ++st, d += 4 * LD) {
-                if (k + 4 * st >= K) break;
-                float2 w[MW];
-#pragma unroll
-                for (int q = 0; q < MW; ++q) {
-                    w[q] = s_tw[i[q]];
-                    i[q] += t[q];
-                    i[q] -= i[q] >= G ? G : 0;
-                }
-                const float ar = d[0], ai = d[CT], br = d[2 * CT], bi = d[3 * CT];
-#pragma unroll
-                for (int q = 0; q < MW; ++q) {
-                    part[q][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, w[q].x, part[q][0], 0, 0, 0);
-                    part[q][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, w[q].x, part[q][1], 0, 0, 0);
-                    part[q][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(br, w[q].y, part[q][2], 0, 0, 0);
-                    part[q][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(bi, w[q].y, part[q][3], 0, 0, 0);
-                }
+            for (int q = 0; q < MW; ++q) {
+                w[q] = s_tw[i[q]];
+                i[q] += t[q];
+                i[q] -= i[q] >= G ? G : 0;
             }
+            const float ar = d[0], ai = d[CT], br = d[2 * CT], bi = d[3 * CT];
+            d += 4 * LD;
+#pragma unroll
+            for (int q = 0; q < MW; ++q) {
+                part[q][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, w[q].x, part[q][0], 0, 0, 0);
+                part[q][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, w[q].x, part[q][1], 0, 0, 0);
+                part[q][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(br, w[q].y, part[q][2], 0, 0, 0);
+                part[q][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(bi, w[q].y, part[q][3], 0, 0, 0);
+            }
+        };
+        auto add = [&]() {
 #pragma unroll
             for (int q = 0; q < MW; ++q)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[q][j] += part[q][j];
+        };
+        int k = 0;
+        for (; k + 16 <= K; k += 16) {
+            clear();
+#pragma unroll
+            for (int st = 0; st < 4; ++st) step();
+            add();
+        }
+        if (k < K) {
+            clear();
+            for (; k < K; k += 4) step();
+            add();
         }
 #pragma unroll
         for (int q = 0; q < MW; ++q) {
@@ -1947,7 +1962,7 @@ __device__ __forceinline__ void dft_product(const float* s_d, const float2* s_tw
                 pos[r] = make_float2(acc[q][0][r] - acc[q][3][r], acc[q][1][r] + acc[q][2][r]);
                 neg[r] = make_float2(acc[q][0][r] + acc[q][3][r], acc[q][1][r] - acc[q][2][r]);
             }
-            store(m[q], cb * 16 + 4 * kk, pos, neg);
+            store(m[q], cb * 16 + 2 * kk, pos, neg);
         }
     }
 }
@@ -2000,20 +2015,20 @@ __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftcol(int G, int N, i
     float2* dst = out + o * (int64_t)orows * I + i0;
     const int left = (int)std::min<int64_t>(CT, I - i0);
     auto put = [&](int row, int c0, const float2* v) {
-        float2* d = dst + (int64_t)row * I + c0;
+        float2* d = dst + (int64_t)row * I;
         float2 x[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+            const int c = c0 + 4 * (r & 2) + (r & 1);
             x[r] = v[r];
             if (CART)
-                x[r] = c_scale(x[r], FWD ? e.factor * (c0 + r < left ? cmask(e, o, G, row, I, i0 + c0 + r) : 0.f) : e.factor);
+                x[r] = c_scale(x[r], FWD ? e.factor * (c < left ? cmask(e, o, G, row, I, i0 + c) : 0.f) : e.factor);
         }
-        if (c0 + 4 <= left) {
-            __builtin_memcpy(d, x, 32);
-        } else {
 #pragma unroll
-            for (int r = 0; r < 3; ++r)
-                if (c0 + r < left) d[r] = x[r];
+        for (int r = 0; r < 4; r += 2) {
+            const int c = c0 + 4 * r;
+            if (c + 2 <= left) __builtin_memcpy(d + c, x + r, 16);
+            else if (c < left) d[c] = x[r];
         }
     };
     dft_product<CT, MW>(s_d, s_tw, K, M, G, [&](int m, int c0, const float2* pos, const float2* neg) {
@@ -2037,7 +2052,8 @@ __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftcol(int G, int N, i
 template <bool FWD, int CT, int MW>
 __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftrow(Geo g, Batch bt, int G, const float2* __restrict__ twg,
                                                 const float* __restrict__ apod, const float2* __restrict__ in,
-                                                float2* __restrict__ out, int KC, int YG, int nkc, int l0, float factor) {
+                                                float2* __restrict__ out, int KC, int YG, int nkc, int l0, float factor,
+                                                uint64_t km) {
     extern __shared__ __attribute__((aligned(16))) float2 sh[];
     __shared__ int64_t s_img[CT], s_grid[CT];  // the lines' image offset (-1: none) and grid offset
     __shared__ int64_t s_map[CT];              // field-map offset of the line (-1: none)
@@ -2082,30 +2098,30 @@ __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftrow(Geo g, Batch bt
     }
     __syncthreads();
     if (FWD) {
-        // 32 lanes along the image row, 8 lines at a time
-        const int kl = threadIdx.x & 31;
-        for (int c = threadIdx.x >> 5; c < CT; c += blockDim.x >> 5) {
+        // lanes along the image row, then over the lines; 8 loads in flight per lane
+        const int k4 = dft_k4(K), total = k4 * CT;
+#pragma unroll 4
+        for (int q0 = threadIdx.x; q0 < total; q0 += blockDim.x) {
+            const int c = mdiv(q0, km), k = q0 - c * k4;
             const int64_t im = s_img[c], mp = s_map[c];
             const float ap = s_ap[c];
             auto load = [&](int p) {
                 float2 x = c_scale(in[im + p], ap * apx[p]);
                 return mp >= 0 ? c_mul(x, bt.b0s[mp + p]) : x;
             };
-#pragma unroll 2
-            for (int k = kl; k < dft_k4(K); k += 32) {
-                float2 p = make_float2(0.f, 0.f), q = p;
-                if (im >= 0 && k < hp) p = load(h + k);
-                if (im >= 0 && k >= 1 && k <= h) q = load(h - k);
-                dft_put<CT>(s_d, k, c, p, q);
-            }
+            float2 p = make_float2(0.f, 0.f), q = p;
+            if (im >= 0 && k < hp) p = load(h + k);
+            if (im >= 0 && k >= 1 && k <= h) q = load(h - k);
+            dft_put<CT>(s_d, k, c, p, q);
         }
     } else {
         // lanes along the values when a grid point holds several of them, else along the row
         const bool vmaj = KC >= 4;
-        const int total = dft_k4(K) * CT;
-#pragma unroll 2
+        const int k4 = dft_k4(K), total = k4 * CT;
+#pragma unroll 4
         for (int q0 = threadIdx.x; q0 < total; q0 += blockDim.x) {
-            const int c = vmaj ? q0 % CT : q0 / dft_k4(K), k = vmaj ? q0 / CT : q0 % dft_k4(K);
+            const int qk = mdiv(q0, km);
+            const int c = vmaj ? q0 % CT : qk, k = vmaj ? q0 / CT : q0 - qk * k4;
             const float2* src = in + s_grid[c];
             float2 p = make_float2(0.f, 0.f), q = p;
             if (s_img[c] >= 0) {
@@ -2117,28 +2133,28 @@ __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftrow(Geo g, Batch bt
     }
     __syncthreads();
     if (FWD) {
-        const bool quads = KC % 4 == 0;  // a lane's 4 lines are 4 neighbouring values
+        const bool pairs = KC % 2 == 0 && VT % 2 == 0;  // lines c0, c0 + 1 are neighbouring values
         dft_product<CT, MW>(s_d, s_tw, K, M, G, [&](int m, int c0, const float2* pos, const float2* neg) {
             const bool both = m >= 1 && 2 * m < G;
-            if (quads && s_img[c0 + 3] >= 0) {
-                float2* d = out + s_grid[c0];
-                __builtin_memcpy(d + m * RC, pos, 32);
-                if (both) __builtin_memcpy(d + (G - m) * RC, neg, 32);
-                return;
-            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                if (s_img[c0 + r] < 0) continue;
-                float2* d = out + s_grid[c0 + r];
-                d[m * RC] = pos[r];
-                if (both) d[(G - m) * RC] = neg[r];
+                const int c = c0 + 4 * (r & 2) + (r & 1);
+                if (s_img[c] < 0) continue;
+                float2* d = out + s_grid[c];
+                if (!pairs) {
+                    d[m * RC] = pos[r];
+                    if (both) d[(G - m) * RC] = neg[r];
+                } else if (r % 2 == 0) {
+                    __builtin_memcpy(d + m * RC, pos + r, 16);
+                    if (both) __builtin_memcpy(d + (G - m) * RC, neg + r, 16);
+                }
             }
         });
     } else {
         dft_product<CT, MW>(s_d, s_tw, K, M, G, [&](int m, int c0, const float2* pos, const float2* neg) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int c = c0 + r;
+                const int c = c0 + 4 * (r & 2) + (r & 1);
                 const int64_t im = s_img[c], mp = s_map[c];
                 if (im < 0) continue;
                 auto put = [&](int p, float2 x) {
@@ -2157,27 +2173,26 @@ __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftrow(Geo g, Batch bt
 // sides, in place
 template <bool FWD, int CT, int MW>
 __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftcartrow(int G, int64_t nrows, const float2* __restrict__ twg, const float2* in,
-                                                    float2* out, CartEpi e) {
+                                                    float2* out, CartEpi e, uint64_t km) {
     extern __shared__ __attribute__((aligned(16))) float2 sh[];
     float2* s_tw = sh;
     float* s_d = reinterpret_cast<float*>(sh + G);
     const int64_t r0 = (int64_t)pf_xcd_remap(blockIdx.x, gridDim.x) * CT;
     const int h = G / 2, hp = G - G / 2, K = h + 1;
     for (int i = threadIdx.x; i < G; i += blockDim.x) s_tw[i] = twg[i];
-    const int kl = threadIdx.x & 31;
-    for (int c = threadIdx.x >> 5; c < CT; c += blockDim.x >> 5) {
+    const int k4 = dft_k4(K), total = k4 * CT;
+#pragma unroll 4
+    for (int q0 = threadIdx.x; q0 < total; q0 += blockDim.x) {
+        const int c = mdiv(q0, km), k = q0 - c * k4;
         const int64_t row = r0 + c;
         auto load = [&](int j) {
             const float2 x = in[row * G + j];
             return FWD ? x : c_scale(x, cmask(e, row, 1, 0, G, j));
         };
-#pragma unroll 2
-        for (int k = kl; k < dft_k4(K); k += 32) {
-            float2 p = make_float2(0.f, 0.f), q = p;
-            if (row < nrows && k < hp) p = load(h + k);
-            if (row < nrows && k >= 1 && k <= h) q = load(h - k);
-            dft_put<CT>(s_d, k, c, p, q);
-        }
+        float2 p = make_float2(0.f, 0.f), q = p;
+        if (row < nrows && k < hp) p = load(h + k);
+        if (row < nrows && k >= 1 && k <= h) q = load(h - k);
+        dft_put<CT>(s_d, k, c, p, q);
     }
     __syncthreads();
     dft_product<CT, MW>(s_d, s_tw, K, K, G, [&](int m, int c0, const float2* pos, const float2* neg) {
@@ -2185,7 +2200,7 @@ __global__ void __launch_bounds__(MW == 1 ? 1024 : 256) k_dftcartrow(int G, int6
         const float2* dn = FWD ? neg : pos;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int64_t row = r0 + c0 + r;
+            const int64_t row = r0 + c0 + 4 * (r & 2) + (r & 1);
             if (row >= nrows) continue;
             auto put = [&](int j, float2 x) {
                 out[row * G + j] = c_scale(x, FWD ? e.factor * cmask(e, row, 1, 0, G, j) : e.factor);
@@ -2308,6 +2323,14 @@ int pf_fftk_init(pf_plan* p) {
             reinterpret_cast<const void*>(k_dftcol<false, 32, 2, true>),
             reinterpret_cast<const void*>(k_dftrow<false, 32, 2>),
             reinterpret_cast<const void*>(k_dftcartrow<false, 32, 2>),
+            reinterpret_cast<const void*>(k_dftcol<true, 32, 1, false>),
+            reinterpret_cast<const void*>(k_dftcol<true, 32, 1, true>),
+            reinterpret_cast<const void*>(k_dftrow<true, 32, 1>),
+            reinterpret_cast<const void*>(k_dftcartrow<true, 32, 1>),
+            reinterpret_cast<const void*>(k_dftcol<false, 32, 1, false>),
+            reinterpret_cast<const void*>(k_dftcol<false, 32, 1, true>),
+            reinterpret_cast<const void*>(k_dftrow<false, 32, 1>),
+            reinterpret_cast<const void*>(k_dftcartrow<false, 32, 1>),
             reinterpret_cast<const void*>(k_dftcol<true, 16, 2, false>),
             reinterpret_cast<const void*>(k_dftcol<true, 16, 2, true>),
             reinterpret_cast<const void*>(k_dftrow<true, 16, 2>),
@@ -2413,7 +2436,10 @@ static int dft_shape(const pf_fftk_axis& X, bool fwd, bool split, Blocks&& block
     d.K = fwd ? h : half;
     const int M = fwd ? half : h;
     d.CT = dft_ct(d.K);
-    d.MW = 2;
+    // output pairs per wave step: 32 share each row read, 16 leave fewer idle
+    // waves in the last round of 4
+    const int u16 = (M + 15) / 16 * (d.CT / 16), u32 = (M + 31) / 32 * (d.CT / 16);
+    d.MW = (u16 + 3) / 4 < 2 * ((u32 + 3) / 4) ? 1 : 2;
     d.threads = 256;
     int64_t nblk = blocks(d.CT), parts = 1;
     if (nblk < 512) {
@@ -2439,8 +2465,9 @@ static int launch_dft_col(const pf_fftk_axis& X, bool fwd, bool cart, int64_t O,
     if (rc != PF_OK || d.grid.x < 1) return rc;
 #define PF_DFTCOL(F, T, W, C) \
     hipLaunchKernelGGL((k_dftcol<F, T, W, C>), d.grid, dim3(d.threads), d.lds, s, X.G, X.N, I, X.tw, src, dst, cm, e)
-#define PF_DFTCOL2(F, C)                          \
-    if (d.CT == 32) PF_DFTCOL(F, 32, 2, C);       \
+#define PF_DFTCOL2(F, C)                                   \
+    if (d.CT == 32 && d.MW == 2) PF_DFTCOL(F, 32, 2, C);   \
+    else if (d.CT == 32) PF_DFTCOL(F, 32, 1, C);           \
     else if (d.MW == 2) PF_DFTCOL(F, 16, 2, C);   \
     else PF_DFTCOL(F, 16, 1, C)
     if (cart && fwd) {
@@ -2479,9 +2506,10 @@ static int launch_dft_row(const pf_plan* p, const pf_batch& b, bool fwd, const f
     const Batch t = batch_of(b);
 #define PF_DFTROW(F, T, W, L0, FAC)                                                                                  \
     hipLaunchKernelGGL((k_dftrow<F, T, W>), d.grid, dim3(d.threads), d.lds, s, g, t, X.G, X.tw, p->apod, src, dst, KC, YG, \
-                       nkc, L0, FAC)
-#define PF_DFTROW2(F, L0, FAC)                          \
-    if (d.CT == 32) PF_DFTROW(F, 32, 2, L0, FAC);       \
+                       nkc, L0, FAC, magic_of(dft_k4(d.K)))
+#define PF_DFTROW2(F, L0, FAC)                                   \
+    if (d.CT == 32 && d.MW == 2) PF_DFTROW(F, 32, 2, L0, FAC);   \
+    else if (d.CT == 32) PF_DFTROW(F, 32, 1, L0, FAC);           \
     else if (d.MW == 2) PF_DFTROW(F, 16, 2, L0, FAC);   \
     else PF_DFTROW(F, 16, 1, L0, FAC)
     if (fwd) {
@@ -2503,9 +2531,11 @@ static int launch_dft_cartrow(const pf_fftk_axis& X, bool fwd, int64_t nrows, co
     const int rc = dft_shape(X, fwd, src != dst, [&](int CT) { return (nrows + CT - 1) / CT; }, d);
     if (rc != PF_OK || d.grid.x < 1) return rc;
 #define PF_DFTCROW(F, T, W) \
-    hipLaunchKernelGGL((k_dftcartrow<F, T, W>), d.grid, dim3(d.threads), d.lds, s, X.G, nrows, X.tw, src, dst, e)
-#define PF_DFTCROW2(F)                       \
-    if (d.CT == 32) PF_DFTCROW(F, 32, 2);    \
+    hipLaunchKernelGGL((k_dftcartrow<F, T, W>), d.grid, dim3(d.threads), d.lds, s, X.G, nrows, X.tw, src, dst, e, \
+                       magic_of(dft_k4(d.K)))
+#define PF_DFTCROW2(F)                                \
+    if (d.CT == 32 && d.MW == 2) PF_DFTCROW(F, 32, 2); \
+    else if (d.CT == 32) PF_DFTCROW(F, 32, 1);         \
     else if (d.MW == 2) PF_DFTCROW(F, 16, 2); \
     else PF_DFTCROW(F, 16, 1)
     if (fwd) {

@@ -7,17 +7,22 @@
 
 namespace {
 
+// threads per block: the forward gather takes an item's lanes at once (a window
+// of more samples than lanes is staged once per item, so more lanes restage
+// less: 512 against 256, 3-D 256^3 grid x 32 coils, W = 6 2476 -> 2284 us; x 8 coils, W = 4 400 -> 320 us); the
+// derivative gather's registers allow 256: it runs over the items' halves
 constexpr int GCOL_TB = PF_GCOL_MAXS;
+constexpr int GCOL_GTB = PF_GCOL_MAXS / 2;
 constexpr int GCOL_OUT = 4;  // coil pairs per output store of the forward gather
 
-template <int W>
+template <int W, int TB = GCOL_TB>
 struct GColShape {
     static constexpr int DZ = pf_gather_dz(W);
     static constexpr int NPL = DZ + W - 1;                          // staged z planes
     static constexpr int PX = PF_GCOL + W - 1;                       // staged points per y and x
     static constexpr int PP = PX * PX;
     static constexpr int NPTS = NPL * PP;
-    static constexpr int NK = (NPTS + GCOL_TB - 1) / GCOL_TB;       // staged points per thread
+    static constexpr int NK = (NPTS + TB - 1) / TB;       // staged points per thread
 };
 
 // 16 bytes global -> LDS for each active lane (the destination is the wave's

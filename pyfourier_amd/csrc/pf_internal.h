@@ -83,7 +83,7 @@ static inline const pf_sitems& pf_sitems_for(const pf_slist& L, int V) { return 
 #define PF_GCOL 16
 #endif
 #ifndef PF_GCOL_MAXS
-#define PF_GCOL_MAXS 256  // lanes per work item (one sample each, one block)
+#define PF_GCOL_MAXS 512  // lanes per work item (one sample each)
 #endif
 // z planes per window: (DZ + W - 1) * (PF_GCOL + W - 1)^2 points of 16 bytes
 // within 80 KB (two blocks per CU).  Deeper windows restage less halo per
@@ -99,6 +99,8 @@ struct pf_glist {
     int32_t* ids = nullptr;  // lane slots: sorted-sample index t or -1, PF_GCOL_MAXS per item
     int4* items = nullptr;   // (key, first lane slot, 0, 0)
     int nitems = 0;
+    int4* halves = nullptr;  // the items' halves of PF_GCOL_MAXS / 2 lanes that hold samples (behind the items)
+    int nhalves = 0;
     int ncol[2] = {0, 0};    // columns along y, x
     int nzw = 0;             // z windows
 };

@@ -728,7 +728,7 @@ static int build_glist(pf_plan* p, const TapParams& P, hipStream_t stream) {
     PF_HIP(hipMemcpyAsync(hb.data(), bvals.p, M * 4, hipMemcpyDeviceToHost, stream));  // indexed by t
     PF_HIP(hipStreamSynchronize(stream));
     std::vector<int32_t> lanes, hbs;
-    std::vector<int4> items;
+    std::vector<int4> items, halves;
     lanes.reserve((size_t)M + M / 4);
     for (int64_t e0 = 0; e0 < M;) {
         int64_t e1 = e0;
@@ -744,6 +744,7 @@ static int build_glist(pf_plan* p, const TapParams& P, hipStream_t stream) {
         lanes.resize(l0 + nit * PF_GCOL_MAXS, -1);
         for (size_t k = 0; k < nit; ++k)
             items.push_back(make_int4((int)hk[e0], (int)(l0 + k * PF_GCOL_MAXS), 0, 0));
+        for (size_t k = 0; k < nl; k += PF_GCOL_MAXS / 2) halves.push_back(make_int4((int)hk[e0], (int)(l0 + k), 0, 0));
         e0 = e1;
     }
     if ((int64_t)lanes.size() >= (1ll << 31)) return PF_OK;
@@ -751,11 +752,14 @@ static int build_glist(pf_plan* p, const TapParams& P, hipStream_t stream) {
     for (int32_t v : lanes) placed += v >= 0;
     if (placed != M) return pf_fail(PF_ERR_ARG, "gather lane assignment lost samples (internal error)");
     L.nitems = (int)items.size();
+    L.nhalves = (int)halves.size();
+    items.insert(items.end(), halves.begin(), halves.end());
     PF_HIP(hipMalloc(&L.ids, std::max<size_t>(1, lanes.size()) * sizeof(int32_t)));
     PF_HIP(hipMemcpy(L.ids, lanes.data(), lanes.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     PF_HIP(hipMalloc(&L.items, std::max<size_t>(1, items.size()) * sizeof(int4)));
     if (!items.empty())
         PF_HIP(hipMemcpy(L.items, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice));
+    L.halves = L.items + L.nitems;
     return PF_OK;
 }
 
