@@ -9,7 +9,8 @@ namespace {
 
 // threads per block: the forward gather takes an item's lanes at once (a window
 // of more samples than lanes is staged once per item, so more lanes restage
-// less: 512 against 256, 3-D 256^3 grid x 32 coils, W = 6 2476 -> 2284 us; x 8 coils, W = 4 400 -> 320 us); the
+// less: 512 against 256, 3-D 256^3 grid x 32 coils, W = 6 2476 -> 2300 us, and 2190 us
+// with the items dealt to the XCDs in chunks; x 8 coils, W = 4 400 -> 320 us); the
 // derivative gather's registers allow 256: it runs over the items' halves
 constexpr int GCOL_TB = PF_GCOL_MAXS;
 constexpr int GCOL_GTB = PF_GCOL_MAXS / 2;

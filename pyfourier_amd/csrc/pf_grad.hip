@@ -365,7 +365,7 @@ __global__ void __launch_bounds__(GCOL_GTB, 2)
                         const float2* __restrict__ h, float* __restrict__ dout, int ncy, int ncx, int nzw) {
     using S = GColShape<W, GCOL_GTB>;
     __shared__ float4 win[S::NPTS];
-    const unsigned bid = pf_xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned bid = pf_xcd_deal(blockIdx.x, gridDim.x);
     const int4 it = items[bid];
     const int zw = it.x % nzw;
     const int cx = (it.x / nzw) % ncx;

@@ -259,6 +259,18 @@ __device__ __forceinline__ unsigned pf_xcd_remap(unsigned b, unsigned nb) {
     return base + i;
 }
 
+// The same in chunks of 32 logical blocks dealt to the XCDs in turn, for lists
+// whose work varies along the order (windows and tiles around the k-space
+// centre are fuller): a contiguous eighth each leaves some XCDs with the heavy
+// part, chunks even it out and still keep neighbours on one L2.
+__device__ __forceinline__ unsigned pf_xcd_deal(unsigned b, unsigned nb) {
+    constexpr unsigned CH = 32;
+    const unsigned full = nb / (8 * CH) * (8 * CH);
+    if (b >= full) return full + pf_xcd_remap(b - full, nb - full);
+    const unsigned x = b % 8, i = b / 8;
+    return (i / CH * 8 + x) * CH + i % CH;
+}
+
 // plan helpers shared by the NUFFT and Toeplitz objects
 int pf_plan_params(pf_plan* p, int ndim, const int* shape_zyx, const int* width_zyx,
                    const float* oversamp_zyx, int nframes, int64_t npts, const int* tile_zyx, int chunk);

@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(GCOL_TB, 2)
                  int ncx, int nzw) {
     using S = GColShape<W>;
     __shared__ float4 win[S::NPTS];  // staged window, one coil pair
-    const unsigned bid = pf_xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned bid = pf_xcd_deal(blockIdx.x, gridDim.x);
     const int4 it = items[bid];
     const int zw = it.x % nzw;
     const int cx = (it.x / nzw) % ncx;
@@ -1033,7 +1033,7 @@ template <int TZ, int TY, int TX, int VL>
 __global__ void __launch_bounds__(64, VL == 32 ? 2 : (VL == 16 ? 3 : 4))
     k_spread_pipe(GeoParams g, BatchParams B, const int4* __restrict__ items, const int32_t* __restrict__ slist,
                   const float* __restrict__ taprec, const float2* __restrict__ ys, float2* __restrict__ grid,
-                  float2* __restrict__ partial) {
+                  float2* __restrict__ partial, bool deal) {
     constexpr int EB = SPIPE_EB;
     constexpr bool SMALL = VL < 8;
     constexpr bool SKIP = spipe_small<TZ, TY, TX>();  // row block = one slow-axis position
@@ -1057,7 +1057,7 @@ __global__ void __launch_bounds__(64, VL == 32 ? 2 : (VL == 16 ? 3 : 4))
 
     const int C = B.C;
     const int nvch = (C + VL - 1) / VL;
-    const unsigned bid = pf_xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned bid = deal ? pf_xcd_deal(blockIdx.x, gridDim.x) : pf_xcd_remap(blockIdx.x, gridDim.x);
     const unsigned item = bid / (unsigned)nvch;
     const int4 it = items[item];
     const int vch = (int)(bid - item * (unsigned)nvch);
@@ -2082,8 +2082,14 @@ void launch_reg(dim3 grid, hipStream_t s, const GeoParams& g, const BatchParams&
 template <int TZ, int TY, int TX, int VL>
 void launch_pipe(dim3 grid, hipStream_t s, const GeoParams& g, const BatchParams& B, const pf_slist& L,
                  const pf_sitems& I, const pf_plan* p, const float2* ys, float2* out, float2* partial, const float*) {
+    // items dealt to the XCDs in chunks while the grid fits the 256 MB Infinity
+    // Cache (spread: 113 x 128 x 138 grid x 6 coils 142 -> 120 us, uneven batch
+    // of 2-D slices 181 -> 165 us, 512^2 x 32 values 220 -> 204 us); a larger grid
+    // is bound by its writes, which run faster as one contiguous eighth per XCD
+    // (256^3 x 8 coils 435 -> 411 us)
+    const bool deal = (double)B.nfg * B.C * g.gtot * sizeof(float2) <= 256.0 * (1 << 20);
     hipLaunchKernelGGL((k_spread_pipe<TZ, TY, TX, VL>), grid, dim3(64), 0, s, g, B, I.sitems, L.slist, p->taprec, ys,
-                       out, partial);
+                       out, partial, deal);
 }
 
 template <int TZ, int TY, int TX>
