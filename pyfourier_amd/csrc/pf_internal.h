@@ -232,6 +232,11 @@ bool pf_fftk_masked(const pf_plan* p);
 int pf_fftk_forward(pf_plan* p, const pf_batch& b, const float2* img, float2* grid, float2* extra, hipStream_t s);
 int pf_fftk_adjoint(pf_plan* p, const pf_batch& b, float2* grid, float2* img, float2* extra, float factor,
                     hipStream_t s, bool masked = false);
+// one-kernel Gram: forward passes, the last axis with the pointwise kernel
+// (nfg, Gtot) and back in one pass, inverse passes; where supported
+bool pf_fftk_gram_supported(const pf_plan* p, const pf_batch& b);
+int pf_fftk_gram(pf_plan* p, const pf_batch& b, const float2* img, float2* out, float2* grid, float2* extra,
+                 const float2* kern, float factor, hipStream_t s);
 // masked centred FFT (oversampling 1) on the layout (planes, Nz, Ny, Nx):
 // src -> dst, in place after the first pass; mask (mframes, Nz*Ny*Nx) or null
 int pf_fftk_cart(pf_plan* p, int64_t planes, int T, const float* mask, int mframes, bool fwd, const float2* src,

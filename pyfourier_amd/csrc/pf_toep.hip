@@ -9,7 +9,8 @@
 // NUFFT do the embedding: only rows that hold image data are transformed
 // forward, and the inverse keeps only the N outputs the crop needs.  Between
 // them one kernel applies the per-voxel R x R kernel (R = L segments x K
-// subspace coefficients; R = 1 is a pointwise multiply).  With B0 segments the
+// subspace coefficients; R = 1 on a register line length is multiplied inside
+// the pass along the last axis, k_gramcolq).  With B0 segments the
 // X pass multiplies by Ct_l on the way in and sums conj(Ct_l) on the way out.
 //
 // The same object, built on the N grid itself (oversampling 1, no embedding)
@@ -215,6 +216,9 @@ int pf_toeplitz_apply(pf_toep* t, int batch, const void* image, void* out, const
     float2* grid = static_cast<float2*>(workspace);
     float2* extra = reinterpret_cast<float2*>(static_cast<char*>(workspace) + gb);
     const bool fused = pf_fftk_supported(t->geo);
+    if (pf_fftk_gram_supported(t->geo, b))
+        return pf_fftk_gram(t->geo, b, static_cast<const float2*>(image), static_cast<float2*>(out), grid, extra, t->T,
+                            (float)(1.0 / (double)pf_gtot(t->geo)), s);
     int rc;
     if (fused) {
         rc = pf_fftk_forward(t->geo, b, static_cast<const float2*>(image), grid, extra, s);
