@@ -15,7 +15,7 @@
  *     synchronise once when the object is built (fused-FFT twiddle tables
  *     included), so operator calls may be captured into a HIP graph from the
  *     first one.  One exception: grid sizes with prime factors other than
- *     2, 3 and 5 run rocFFT, whose plan and work buffer for a new batch size
+ *     2, 3 and 5 and more than 1024 points run rocFFT, whose plan and work buffer for a new batch size
  *     are made (under the plan's lock) at the first call with that size.
  *   - Every call returns 0 on success or a PF_ERR_* code; pf_last_error()
  *     returns a thread-local message for the last failure.  Arguments are
@@ -188,8 +188,8 @@ int pf_describe_launch(const pf_plan* plan, const pf_batch_desc* desc, char* buf
  * memory at call time (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same results as pf_nufft /
  * pf_nufft_adj.  Limits: the call's pf_workspace_size must not exceed
- * PF_NOALLOC_SCRATCH_BYTES and the grid sizes must be 2^a 3^b 5^c (rocFFT
- * sizes allocate), else PF_ERR_UNSUPPORTED before any launch; the current
+ * PF_NOALLOC_SCRATCH_BYTES and the grid sizes must be 2^a 3^b 5^c
+ * or 7-smooth register sizes, else PF_ERR_UNSUPPORTED before any launch; the current
  * device must be the plan's.  Every call on one GPU shares its array:
  * calls that overlap in time on one GPU (other streams, other threads)
  * race and must be serialised by the caller. */
@@ -236,7 +236,9 @@ int pf_workspace_offsets(const pf_plan* plan, const pf_batch_desc* desc, size_t*
 /* Fused deapodise + zero-pad + centred FFT: image (C, nimg, N...) -> grid.
  * For grid sizes 2^a 3^b 5^c, and the 7-smooth sizes 112, 224, 280, 336 and
  * 448 (<= 4096 per axis), a pruned FFT transforms only the lines that hold
- * image data; otherwise pf_deapod_pad + pf_fft.  On the 7-smooth sizes a
+ * image data; other
+ * lengths up to 1024 do so with a dense DFT; otherwise pf_deapod_pad +
+ * pf_fft.  On the 7-smooth sizes a
  * batch takes at most 16 field-map segments per call.
  * Replaces src/pyfourier/_nufft/_nufft.py:234-241.  fft_workspace: the FFT
  * scratch part of the pf_nufft workspace (pf_workspace_offsets).  Grid
@@ -293,7 +295,8 @@ typedef struct pf_toep pf_toep;
  *         (index order of an uncentred FFT), already scaled as the operator
  *         needs; copied into the object.  R <= PF_TOEP_RMAX.
  * shape:  host (ndim,) image matrix N (z, y, x).  Embedding sizes 2^a 3^b 5^c
- *         (<= 4096 per axis) run the pruned fused FFT passes, others rocFFT. */
+ *         (<= 4096 per axis) and others up to 1024 run the pruned fused FFT
+ *         passes, the rest rocFFT. */
 int pf_toeplitz_create(const void* kernel, int ndim, const int* shape, int nseg, int ncoeff, void* stream,
                        pf_toep** out);
 int pf_toeplitz_destroy(pf_toep* op);
@@ -319,7 +322,7 @@ int pf_toeplitz_apply(pf_toep* op, int batch, const void* image, void* out, cons
  * nframes: kernels per image frame (1 with a basis); the image is then
  *         (batch, nframes, N...), or (batch, ncoeff, N...) with a basis.
  * shape:  host (ndim,) N (z, y, x); sizes with prime factors other than 2, 3
- *         and 5 use rocFFT. */
+ *         and 5 above 1024 use rocFFT. */
 int pf_gram_create(const void* kernel, int ndim, const int* shape, int nframes, int nseg, int ncoeff,
                    void* stream, pf_toep** out);
 
@@ -335,7 +338,7 @@ typedef struct pf_cart pf_cart;
  *        mask; copied.  mframes is 1 (shared by every frame) or the frame
  *        count of the calls.
  * shape: host (ndim,) matrix (z, y, x).  Sizes that factor into 2, 3, 5 use
- *        the fused FFT passes, other sizes rocFFT. */
+ *        the fused FFT passes, as do others up to 1024; the rest rocFFT. */
 int pf_cart_create(const float* mask, int mframes, int ndim, const int* shape, void* stream, pf_cart** out);
 int pf_cart_destroy(pf_cart* plan);
 

@@ -98,7 +98,7 @@ WsLayout layout(const pf_plan* p, const pf_batch& b) {
 }
 
 // FFT state a plan needs before its first operator call: the fused pruned
-// FFT's twiddle tables for grid sizes 2^a 3^b 5^c (built here, so calls
+// FFT's twiddle tables for the grid sizes it takes (built here, so calls
 // neither allocate nor synchronise), otherwise the rocFFT plan cache, whose
 // per-batch-size rocFFT plans are made on first use under its lock.
 int plan_fft_state(pf_plan* p) {

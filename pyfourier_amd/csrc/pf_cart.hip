@@ -14,7 +14,7 @@
 // mask and norm factor fused into the last forward / first inverse pass and
 // no workspace (pf_fftk_cart).  Otherwise the object's sample-free geometry
 // plan (width 1, oversampling 1, unit apodisation) lets the fused FFT passes
-// of the NUFFT (or rocFFT for sizes with other prime factors) compute FFTc on
+// of the NUFFT (or rocFFT for sizes it does not take) compute FFTc on
 // the (nfg, Cb, Nz, Ny, Nx, R, Cv) grid in stored FFT order.  One more kernel per direction moves between that grid and
 // the caller's (C, T, Nz, Ny, Nx) centred k-space: it applies the shift, the
 // basis contraction over K, the B0 sum over L, the mask and the norm factor in

@@ -142,8 +142,8 @@ struct pf_plan {
     int max_chunk = 0;    // spread entries per work item (0: automatic)
     pf_glist gl;          // LDS-staged gather lists (empty when not built)
 
-    pf_fft_cache* fft = nullptr;   // rocFFT plans (grid sizes with other prime factors)
-    struct pf_fftk* fftk = nullptr; // fused pruned FFT (sizes 2^a 3^b 5^c)
+    pf_fft_cache* fft = nullptr;   // rocFFT plans (sizes the fused FFT does not take)
+    struct pf_fftk* fftk = nullptr; // fused pruned FFT (pf_fftk_supported)
 };
 
 // ---- error handling --------------------------------------------------------

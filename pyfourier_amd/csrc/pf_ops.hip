@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(GTB) __attribute__((amdgpu_waves_per_eu(1, DEE
 // no basis, no field map; an even batch C).  The forward grid of such a
 // batch is laid out coil-pair major, (nfg, C/2, Gz, Gy, Gx, 2), so one coil
 // pair of a window row is one contiguous run.
-// One block per work item of the plan's gather lists: 256 lanes holding
+// One block per work item of the plan's gather lists: 512 lanes holding
 // samples whose first taps all lie in one window, a PF_GCOL x PF_GCOL column
 // in (y, x) times DZ consecutive z planes (lane order chosen at plan time so
 // that the 16 lanes of an LDS pass mostly read distinct banks).  For each
@@ -2227,7 +2227,6 @@ std::string pf_spread_name(const pf_plan* p, const pf_batch& b) {
     }
     const int VC = pf_spread_coil_chunk(p, b);
     const int V = b.Cb * b.R * b.Cv;
-    const int nvch = (V + VC - 1) / VC;
     if (pf_sitems_for(pf_slist_for(p, b), V).nritems > 0) name += "+k_spread_reduce";
     return name;
 }

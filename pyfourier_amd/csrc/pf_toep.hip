@@ -223,7 +223,7 @@ int pf_toeplitz_apply(pf_toep* t, int batch, const void* image, void* out, const
     if (fused) {
         rc = pf_fftk_forward(t->geo, b, static_cast<const float2*>(image), grid, extra, s);
     } else {
-        // grid sizes with other prime factors: generic pad, rocFFT, crop
+        // sizes the fused FFT does not take: generic pad, rocFFT, crop
         rc = pf_launch_deapod_pad(t->geo, b, static_cast<const float2*>(image), grid, s);
         if (rc == PF_OK) rc = pf_fft_exec(t->geo, b, grid, 0, s);
     }
