@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "../../include/pfhip.h"
+#include "pf_taprec.h"
 
 #define PF_WMAX 8
 

@@ -1116,8 +1116,8 @@ __global__ void __launch_bounds__(64, VL == 32 ? 2 : (VL == 16 ? 3 : 4))
     };
     auto load_data = [&]() {
         const float4* r = reinterpret_cast<const float4*>(taprec) + (int64_t)id_r * rec4;
-        rec0 = r[lane & 3];
-        if (rec4 > 4) rec1 = r[(lane & 3) + 4 < rec4 ? (lane & 3) + 4 : 0];
+        rec0 = r[pf_rec_piece(lane & 3, rec4)];
+        if (rec4 > 4) rec1 = r[pf_rec_piece((lane & 3) + 4, rec4)];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float* y = yf + (int64_t)id_v[j] * (2 * C);
@@ -1360,7 +1360,7 @@ __device__ __forceinline__ void smfma_issue(float4 (&s_rec)[SPIPE_EB][SPIPE_RP],
                                             const char* __restrict__ ybase, int C, int vch) {
     const int lane = threadIdx.x;
     const int c = lane & (SPIPE_RP - 1);
-    const int cs = c < rec4 ? c : 0;
+    const int cs = pf_rec_piece(c, rec4);
 #pragma unroll
     for (int k = 0; k < SPIPE_EB * SPIPE_RP / 64; ++k) {
         const int e = k * (64 / SPIPE_RP) + (lane >> 3);

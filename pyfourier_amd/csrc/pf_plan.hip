@@ -345,7 +345,7 @@ int pf_plan_params(pf_plan* p, int ndim, const int* shape_zyx, const int* width_
         tt = tu;
     }
     p->ntile_tot = 1;
-    int off = 4;
+    int off = PF_REC_HEAD;
     for (int a = 0; a < 3; ++a) {
         p->tile[a] = std::min(tt[a], p->os[a]);
         // a footprint must not leave a tile and re-enter it across the
@@ -358,7 +358,7 @@ int pf_plan_params(pf_plan* p, int ndim, const int* shape_zyx, const int* width_
     }
     if ((int64_t)nframes * p->ntile_tot >= (1ll << 31))
         return pf_fail(PF_ERR_UNSUPPORTED, "too many tiles");
-    p->rec = (off + 3) & ~3;
+    p->rec = pf_rec_words(p->width[0], p->width[1], p->width[2]);
     if (chunk < 0) return pf_fail(PF_ERR_ARG, "chunk must be >= 0 (0: automatic)");
     p->max_chunk = chunk;  // 0: chosen from the spread list size when it is built
     return PF_OK;
