@@ -351,12 +351,13 @@ const GradLaunch DCOORD_W_DEEP[2][PF_WMAX] = {
 // LDS-staged derivative gather for the batches the forward gather stages (3-D,
 // one width W = 3..8 on all axes, plain values, coil-pair-major grid: Cv = 2,
 // Cb = C / 2).  Same work items, lane order and window staging as the forward
-// LDS gather: one block per (frame, 16 x 16 column, DZ z planes) window, one
-// lane per sample, the window of each coil pair copied to LDS and read from
-// there.  Per (z, y) row a lane forms the x-weighted and x-derivative-weighted
-// sums of its W taps and folds them into the three derivatives; Re(conj(h) D)
-// accumulates over the coil pairs in registers, so each sample is written once
-// and no cross-lane reduction is needed.
+// LDS gather, at half its block: one block per half item (256 lanes that hold
+// samples) of a (frame, 16 x 16 column, DZ z planes) window, one lane per
+// sample, the window of each coil pair copied to LDS and read from there.  Per
+// tap a lane forms Re(conj(h) v) over the pair; per (z, y) row the x-weighted and
+// x-derivative-weighted sums of its W taps, folded into the pair's three
+// derivatives, which are added to the sample's once per pair: each sample is
+// written once and no cross-lane reduction is needed.
 template <int W>
 __global__ void __launch_bounds__(GCOL_GTB, 2)
     k_gather_dcoord_col(GradParams P, const int4* __restrict__ items, const int32_t* __restrict__ gids,
@@ -424,8 +425,11 @@ __global__ void __launch_bounds__(GCOL_GTB, 2)
         if (act) {
             // Re(conj(h) v) of each tap first: the sums over taps are then
             // real, 6 operations per tap instead of 8, and a row's fold costs 3
-            // instead of 12
+            // instead of 12.  A pair has its own sums, added to the result once:
+            // one sum running over the W^2 rows of all pairs errs more with
+            // every pair (32 coils, W = 6: 4.3e-7 against 1.5e-7)
             const float4 hv = hp[cp];
+            float sum[3] = {0.f, 0.f, 0.f};
 #pragma unroll
             for (int a = 0; a < W; ++a)
 #pragma unroll
@@ -439,10 +443,12 @@ __global__ void __launch_bounds__(GCOL_GTB, 2)
                         s0 += w[2][c] * t;
                         s1 += dw[2][c] * t;
                     }
-                    part[0] += dw[0][a] * w[1][b] * s0;
-                    part[1] += w[0][a] * dw[1][b] * s0;
-                    part[2] += w[0][a] * w[1][b] * s1;
+                    sum[0] += dw[0][a] * w[1][b] * s0;
+                    sum[1] += w[0][a] * dw[1][b] * s0;
+                    sum[2] += w[0][a] * w[1][b] * s1;
                 }
+#pragma unroll
+            for (int a = 0; a < 3; ++a) part[a] += sum[a];
         }
         __syncthreads();  // the next pair's copies overwrite the window
     }
