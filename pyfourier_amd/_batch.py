@@ -105,6 +105,22 @@ class _Group:
                           _lib.ptr(self.weight), code, _lib.ptr(ws), nbytes, _lib.stream_of(self.device)))
 
 
+def _same_place(a: torch.Tensor, b: torch.Tensor) -> bool:
+    return a.data_ptr() == b.data_ptr() and a.stride() == b.stride() and a.shape == b.shape
+
+
+def _rows_contiguous(d: torch.Tensor, device) -> bool:
+    """complex64 on the device, everything behind the first axis contiguous."""
+    if d.dtype is not torch.complex64 or d.device != device or d.is_conj():
+        return False
+    step = 1
+    for n, st in zip(reversed(d.shape[1:]), reversed(d.stride()[1:])):
+        if n != 1 and st != step:
+            return False
+        step *= n
+    return True
+
+
 class NUFFTBatch:
     """Forward / adjoint NUFFT of an uneven list of problems.
 
@@ -117,7 +133,7 @@ class NUFFTBatch:
     ``images[i]`` (nbatch, nimg_i, *shape_i) and ``kspace[i]`` (nbatch,
     ncontrasts_i, npts_i) are (views of) the static buffers the launches
     read and write: fill them in place, or pass lists to forward/adjoint,
-    which copy with one multi-tensor copy.  A call overwrites the previous
+    which copy with one native launch.  A call overwrites the previous
     results.  group=False runs every item as its own calls (one graph).
     """
 
@@ -230,12 +246,18 @@ class NUFFTBatch:
             if s.numel() != d.numel():
                 raise ValueError(f"item of {s.numel()} values does not fit a buffer of shape {tuple(d.shape)}")
             srcs.append(s.reshape(d.shape).to(device=self.device, dtype=torch.complex64))
-        if torch.is_grad_enabled() and any(s.requires_grad for s in srcs):
-            torch._foreach_copy_(dst, srcs)
-            return
         # one native launch for all items: the buffers are (nbatch, planes or
         # frames, ...) views whose rows (everything behind the batch axis) are
-        # contiguous
+        # contiguous.  Its blocks run in any order, so a source that lies in the
+        # buffers elsewhere than its own place is copied item by item, as are
+        # sources autograd follows and entries a caller replaced by arrays of
+        # another layout
+        bufs = {d.untyped_storage().data_ptr() for d in dst}
+        if ((torch.is_grad_enabled() and any(s.requires_grad for s in srcs))
+                or any(s.untyped_storage().data_ptr() in bufs and not _same_place(s, d) for s, d in zip(srcs, dst))
+                or not all(_rows_contiguous(d, self.device) for d in dst)):
+            torch._foreach_copy_(dst, srcs)
+            return
         srcs = [s.resolve_conj().resolve_neg().contiguous() for s in srcs]
         n = len(dst)
         rows = [int(d.shape[0]) for d in dst]
@@ -245,6 +267,8 @@ class NUFFTBatch:
                 n, (ctypes.c_void_p * n)(*[_lib.ptr(s) for s in srcs]), (ctypes.c_void_p * n)(*[_lib.ptr(d) for d in dst]),
                 LL(*rows), LL(*[d.numel() // max(1, r) for d, r in zip(dst, rows)]), LL(*[int(d.stride(0)) for d in dst]),
                 _lib.stream_of(self.device)))
+        # an in-place write like any other: a graph that saved the old contents must notice
+        torch.autograd.graph.increment_version([d for d in dst if not d.is_inference()])
 
 
 def plan_nufft_batch(coords, shapes, nbatch=1, width=4, oversamp=1.25, weights=None, basis=None, norm=None,
