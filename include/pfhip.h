@@ -187,10 +187,13 @@ int pf_describe_launch(const pf_plan* plan, const pf_batch_desc* desc, char* buf
  * No counterpart in the reference: for callers that cannot allocate device
  * memory at call time (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same results as pf_nufft /
- * pf_nufft_adj.  Limits: the call's pf_workspace_size must not exceed
- * PF_NOALLOC_SCRATCH_BYTES and the grid sizes must be 2^a 3^b 5^c
- * or 7-smooth register sizes, else PF_ERR_UNSUPPORTED before any launch; the current
- * device must be the plan's.  Every call on one GPU shares its array:
+ * pf_nufft_adj, bit for bit where the call's pf_workspace_size fits the
+ * array; a call whose usual workspace does not takes the form that needs
+ * least (field-map and basis coefficients applied while spreading, fewer
+ * partial tiles) and agrees to FP32 rounding.  Limits: that form must fit
+ * PF_NOALLOC_SCRATCH_BYTES and the grid sizes must be 2^a 3^b 5^c or 56,
+ * 112, 168, 224, 280, 336, 448, else PF_ERR_UNSUPPORTED before any launch;
+ * the current device must be the plan's.  Every call on one GPU shares its array:
  * calls that overlap in time on one GPU (other streams, other threads)
  * race and must be serialised by the caller. */
 int pf_nufft_noalloc(pf_plan* plan, const pf_batch_desc* desc, int op, const void* in, void* out,
@@ -228,8 +231,9 @@ int pf_spread_workspace_size(const pf_plan* plan, const pf_batch_desc* desc, siz
  * [grid | tile-sorted samples | FFT scratch | spread partial tiles].  The
  * samples part holds (F*npts, C) for the stage entry points; for a batch
  * with B0 segments or a basis whose nseg*ncoeff*batch values per grid point
- * form one vector (batch <= 64) it is sized (F*npts, nseg*ncoeff*batch),
- * which pf_nufft_adj fills with the coefficient-applied values. */
+ * form one vector (batch <= 64, at most 1024 values) it is sized (F*npts,
+ * nseg*ncoeff*batch), which pf_nufft_adj fills with the coefficient-applied
+ * values, as long as that is below 4 GiB. */
 int pf_workspace_offsets(const pf_plan* plan, const pf_batch_desc* desc, size_t* grid_off,
                          size_t* samples_off, size_t* fft_off, size_t* spread_off);
 

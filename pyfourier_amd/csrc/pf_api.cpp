@@ -298,14 +298,7 @@ int pf_spread_workspace_size(const pf_plan* p, const pf_batch_desc* d, size_t* b
 }
 
 int pf_workspace_size(const pf_plan* p, const pf_batch_desc* d, int op, size_t* bytes) {
-    pf_batch b;
-    int rc = make_batch(p, d, &b, op == 0 ? DIR_FWD : DIR_ANY);
-    if (rc != PF_OK) return rc;
-    if (!bytes) return pf_fail(PF_ERR_ARG, "null output");
-    if (op != 0 && op != 1) return pf_fail(PF_ERR_ARG, "op must be 0 (forward) or 1 (adjoint)");
-    WsLayout w = layout(p, b);
-    *bytes = op == 0 ? w.fwd_total : w.adj_total;
-    return PF_OK;
+    return pf_workspace_bytes(p, d, op, false, bytes);
 }
 
 int pf_deapod_pad(const pf_plan* p, const pf_batch_desc* d, const void* image, void* grid, void* stream) {
@@ -436,11 +429,36 @@ int pf_ifft_crop(pf_plan* p, const pf_batch_desc* d, void* grid, void* image, fl
 
 int pf_nufft(pf_plan* p, const pf_batch_desc* d, const void* image, void* kspace, const float* weight, int norm,
              void* workspace, size_t workspace_bytes, void* stream) {
+    return pf_run_forward(p, d, image, kspace, weight, norm, workspace, workspace_bytes, stream, false);
+}
+
+int pf_nufft_adj(pf_plan* p, const pf_batch_desc* d, const void* kspace, void* image, const float* weight,
+                 int norm, void* workspace, size_t workspace_bytes, void* stream) {
+    return pf_run_adjoint(p, d, kspace, image, weight, norm, workspace, workspace_bytes, stream, false);
+}
+
+}  // extern "C"
+
+int pf_workspace_bytes(const pf_plan* p, const pf_batch_desc* d, int op, bool lean, size_t* bytes) {
+    pf_batch b;
+    int rc = make_batch(p, d, &b, op == 0 ? DIR_FWD : DIR_ANY);
+    if (rc != PF_OK) return rc;
+    if (!bytes) return pf_fail(PF_ERR_ARG, "null output");
+    if (op != 0 && op != 1) return pf_fail(PF_ERR_ARG, "op must be 0 (forward) or 1 (adjoint)");
+    b.lean = lean;
+    WsLayout w = layout(p, b);
+    *bytes = op == 0 ? w.fwd_total : w.adj_total;
+    return PF_OK;
+}
+
+int pf_run_forward(pf_plan* p, const pf_batch_desc* d, const void* image, void* kspace, const float* weight, int norm,
+                   void* workspace, size_t workspace_bytes, void* stream, bool lean) {
     pf_batch b;
     int rc = make_batch(p, d, &b, DIR_FWD);
     if (rc != PF_OK) return rc;
     if (!image || !kspace) return pf_fail(PF_ERR_ARG, "null array");
     if (norm < PF_NORM_NONE || norm > PF_NORM_ADJOINT) return pf_fail(PF_ERR_ARG, "norm must be 0, 1 or 2");
+    b.lean = lean;
     WsLayout w = layout(p, b);
     if (!workspace || workspace_bytes < w.fwd_total) return pf_fail(PF_ERR_ARG, "workspace too small");
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -461,13 +479,14 @@ int pf_nufft(pf_plan* p, const pf_batch_desc* d, const void* image, void* kspace
     return pf_launch_unsort(p, b, ys, static_cast<float2*>(kspace), weight, (float)factor, s);
 }
 
-int pf_nufft_adj(pf_plan* p, const pf_batch_desc* d, const void* kspace, void* image, const float* weight,
-                 int norm, void* workspace, size_t workspace_bytes, void* stream) {
+int pf_run_adjoint(pf_plan* p, const pf_batch_desc* d, const void* kspace, void* image, const float* weight, int norm,
+                   void* workspace, size_t workspace_bytes, void* stream, bool lean) {
     pf_batch b;
     int rc = make_batch(p, d, &b);
     if (rc != PF_OK) return rc;
     if (!image || !kspace) return pf_fail(PF_ERR_ARG, "null array");
     if (norm < PF_NORM_NONE || norm > PF_NORM_ADJOINT) return pf_fail(PF_ERR_ARG, "norm must be 0, 1 or 2");
+    b.lean = lean;
     WsLayout w = layout(p, b);
     if (!workspace || workspace_bytes < w.adj_total) return pf_fail(PF_ERR_ARG, "workspace too small");
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -501,5 +520,3 @@ int pf_nufft_adj(pf_plan* p, const pf_batch_desc* d, const void* kspace, void* i
     if ((rc = pf_fft_exec(p, b, grid, 1, s)) != PF_OK) return rc;
     return pf_launch_crop_deapod(p, b, grid, static_cast<float2*>(image), (float)factor, s);
 }
-
-}  // extern "C"

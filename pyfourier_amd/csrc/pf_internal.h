@@ -50,7 +50,7 @@ struct pf_sitems {
     int nslots = 0;
 };
 
-constexpr int PF_NSPLIT = 4;
+constexpr int PF_NSPLIT = 5;
 constexpr int PF_SLIST_PAD = 16;  // readable ids past the end of a spread list
 
 struct pf_slist {
@@ -58,8 +58,8 @@ struct pf_slist {
     int64_t nslist = 0;
     int4* items = nullptr;       // every split's items, one allocation
     // heavy tiles split for batches of up to 8, 16, 32 and more values per
-    // grid point (pf_split_for); arrays are shared where the item size is
-    // the same
+    // grid point, and as little as any of them is (pf_sitems_for); arrays are
+    // shared where the item size is the same
     pf_sitems split[PF_NSPLIT];
 };
 
@@ -70,9 +70,6 @@ struct pf_slist {
 #define PF_SPREAD_MINCH 64  // smallest work item of the fine split (entries)
 #endif
 
-static inline int pf_split_for(int V) { return V <= 8 ? 0 : (V <= 16 ? 1 : (V <= 32 ? 2 : 3)); }
-// work items of a batch of V values per grid point
-static inline const pf_sitems& pf_sitems_for(const pf_slist& L, int V) { return L.split[pf_split_for(V)]; }
 
 // Gather column lists (3-D plans with one kernel width on all axes): the
 // sorted samples regrouped by window key = (frame, y column, x column, z
@@ -174,7 +171,16 @@ struct pf_batch {
     const float2* b0t;    // (L, nt) temporal interpolator or null
     const float2* b0s;    // (L, Nz*Ny*Nx) spatial maps or null
     int nt;               // readout length for b0t
+    // least workspace: B0 / basis coefficients applied on the fly, the coarsest
+    // spread items.  Set by pf_nufft_noalloc where the usual form does not fit
+    bool lean = false;
 };
+
+// work items of a batch
+static inline const pf_sitems& pf_sitems_for(const pf_slist& L, const pf_batch& b) {
+    const int V = b.Cb * b.R * b.Cv;  // values per grid point
+    return L.split[b.lean ? 4 : (V <= 8 ? 0 : (V <= 16 ? 1 : (V <= 32 ? 2 : 3)))];
+}
 
 // ---- internal launchers (return PF_OK or an error code) -------------------
 int pf_launch_deapod_pad(const pf_plan* p, const pf_batch& b, const float2* img, float2* grid,
@@ -204,6 +210,13 @@ int pf_launch_sort(const pf_plan* p, const pf_batch& b, const float2* y, float2*
 // pipelined spread.  pf_launch_sort_expand then writes the sorted samples as
 // (Mtot, R*C) with the coefficients applied, for pf_launch_spread(bx).
 bool pf_spread_expand(const pf_plan* p, const pf_batch& b, pf_batch* bx);
+
+// bodies of pf_workspace_size, pf_nufft and pf_nufft_adj (pf_api.cpp); lean: pf_batch::lean
+int pf_workspace_bytes(const pf_plan* p, const pf_batch_desc* d, int op, bool lean, size_t* bytes);
+int pf_run_forward(pf_plan* p, const pf_batch_desc* d, const void* image, void* kspace, const float* weight, int norm,
+                   void* workspace, size_t workspace_bytes, void* stream, bool lean);
+int pf_run_adjoint(pf_plan* p, const pf_batch_desc* d, const void* kspace, void* image, const float* weight, int norm,
+                   void* workspace, size_t workspace_bytes, void* stream, bool lean);
 int pf_launch_sort_expand(const pf_plan* p, const pf_batch& b, const float2* y, float2* ys, const float* weight,
                           hipStream_t s);
 int pf_fft_exec(pf_plan* p, const pf_batch& b, float2* grid, int inverse, hipStream_t s);

@@ -53,12 +53,18 @@ extern "C" int pf_nufft_noalloc(pf_plan* p, const pf_batch_desc* d, int op, cons
     if (op != 0 && op != 1) return pf_fail(PF_ERR_ARG, "op must be 0 (forward) or 1 (adjoint)");
     if (!pf_fftk_radix(p))
         return pf_fail(PF_ERR_UNSUPPORTED,
-                       "pf_nufft_noalloc needs grid sizes 2^a 3^b 5^c");
+                       "pf_nufft_noalloc needs grid sizes 2^a 3^b 5^c or 112, 224, 280, 336, 448");
     int dev = -1;
     PF_HIP(hipGetDevice(&dev));
     if (dev != p->device) return pf_fail(PF_ERR_ARG, "the plan lives on another device than the current one");
+    // the usual form, else the one with the least workspace
     size_t need = 0;
-    int rc = pf_workspace_size(p, d, op, &need);
+    bool lean = false;
+    int rc = pf_workspace_bytes(p, d, op, false, &need);
+    if (rc == PF_OK && need > PF_NOALLOC_SCRATCH_BYTES) {
+        lean = true;
+        rc = pf_workspace_bytes(p, d, op, true, &need);
+    }
     if (rc != PF_OK) return rc;
     if (need > PF_NOALLOC_SCRATCH_BYTES)
         return pf_fail(PF_ERR_UNSUPPORTED, "pf_nufft_noalloc: the call needs " + std::to_string(need) +
@@ -70,6 +76,6 @@ extern "C" int pf_nufft_noalloc(pf_plan* p, const pf_batch_desc* d, int op, cons
     if (!ws) return pf_fail(PF_ERR_HIP, "the scratch address lookup failed on this device");
     // nothing in the workspace needs clearing: every kernel writes all of its
     // part (the spread writes every tile of the grid, empty ones as zeros)
-    if (op == 0) return pf_nufft(p, d, in, out, weight, norm, ws, PF_NOALLOC_SCRATCH_BYTES, stream);
-    return pf_nufft_adj(p, d, in, out, weight, norm, ws, PF_NOALLOC_SCRATCH_BYTES, stream);
+    if (op == 0) return pf_run_forward(p, d, in, out, weight, norm, ws, PF_NOALLOC_SCRATCH_BYTES, stream, lean);
+    return pf_run_adjoint(p, d, in, out, weight, norm, ws, PF_NOALLOC_SCRATCH_BYTES, stream, lean);
 }

@@ -2204,7 +2204,7 @@ static size_t spread_tiles_bytes(const pf_plan* p, const pf_batch& b) {
     const int V = b.Cb * b.R * b.Cv;
     const int nvch = (V + VC - 1) / VC;
     const size_t tpts = (size_t)p->tile[0] * p->tile[1] * p->tile[2];
-    return (size_t)pf_sitems_for(pf_slist_for(p, b), V).nslots * nvch * tpts * VC * sizeof(float2);
+    return (size_t)pf_sitems_for(pf_slist_for(p, b), b).nslots * nvch * tpts * VC * sizeof(float2);
 }
 
 std::string pf_spread_name(const pf_plan* p, const pf_batch& b) {
@@ -2225,9 +2225,7 @@ std::string pf_spread_name(const pf_plan* p, const pf_batch& b) {
                    std::to_string(zp) + ">";
         }
     }
-    const int VC = pf_spread_coil_chunk(p, b);
-    const int V = b.Cb * b.R * b.Cv;
-    if (pf_sitems_for(pf_slist_for(p, b), V).nritems > 0) name += "+k_spread_reduce";
+    if (pf_sitems_for(pf_slist_for(p, b), b).nritems > 0) name += "+k_spread_reduce";
     return name;
 }
 
@@ -2259,7 +2257,7 @@ size_t pf_spread_partial_bytes(const pf_plan* p, const pf_batch& b) {
     if (spread_mfma(p, b)) {
         const int nvch = b.C / SPREAD_VL;
         n = al256(n) + al256((size_t)p->mtot * nvch * sizeof(float)) +
-            (size_t)pf_sitems_for(pf_slist_for(p, b), b.C).nsitems * nvch * sizeof(float);
+            (size_t)pf_sitems_for(pf_slist_for(p, b), b).nsitems * nvch * sizeof(float);
     }
     return n;
 }
@@ -2293,7 +2291,7 @@ int pf_launch_spread(const pf_plan* p, const pf_batch& b, const float2* ys, floa
     const size_t lds = spread_lds_bytes(p, VC);
     if (lds > 160 * 1024) return pf_fail(PF_ERR_UNSUPPORTED, "spread tile exceeds LDS");
     const pf_slist& L = pf_slist_for(p, b);
-    pf_sitems I = pf_sitems_for(L, V);
+    pf_sitems I = pf_sitems_for(L, b);
     if (live && I.lsitems) {  // the same items without the empty tiles of uncovered columns
         I.sitems = I.lsitems;
         I.nsitems = I.nlsitems;
@@ -2382,8 +2380,13 @@ int pf_launch_sort(const pf_plan* p, const pf_batch& b, const float2* y, float2*
 constexpr int PF_EXPAND_VMAX = 1024;
 constexpr int PF_EXPAND_QSH = 5;  // 32 samples per block
 
+// The expanded samples take R times the memory of the plain ones: up to 4 GiB of
+// them, and not in a call that is short of workspace; beyond, the spread applies
+// the coefficients on the fly (k_spread_reg).  Measured with it, adjoint, 2-D 256^2,
+// 197k samples, 5 segments x 1 coil 121 -> 67 us, 16 x 64 4196 -> 2793 us.
 bool pf_spread_expand(const pf_plan* p, const pf_batch& b, pf_batch* bx) {
-    if (!PF_SPREAD_EXPAND || (!b.b0t && !b.basis) || b.Cb != 1 || b.R * b.C > PF_EXPAND_VMAX) return false;
+    if (!PF_SPREAD_EXPAND || b.lean || (!b.b0t && !b.basis) || b.Cb != 1 || b.R * b.C > PF_EXPAND_VMAX) return false;
+    if ((uint64_t)p->mtot * b.R * b.C * sizeof(float2) >= (1ull << 32)) return false;
     pf_batch e = b;
     e.C = e.Cv = b.R * b.C;
     e.Cb = 1;
