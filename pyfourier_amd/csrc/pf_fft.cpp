@@ -30,6 +30,7 @@ struct pf_fft_cache {
 
 static std::once_flag g_rocfft_once;
 static rocfft_status g_rocfft_setup = rocfft_status_success;
+static std::mutex g_create_mu;  // creation of a plan's cache
 
 void pf_fft_destroy(pf_fft_cache* c) {
     if (!c) return;
@@ -44,18 +45,18 @@ void pf_fft_destroy(pf_fft_cache* c) {
 int pf_fft_cache_init(pf_plan* p) {
     std::call_once(g_rocfft_once, [] { g_rocfft_setup = rocfft_setup(); });
     if (g_rocfft_setup != rocfft_status_success) return pf_fail(PF_ERR_FFT, "rocfft_setup failed");
+    std::lock_guard<std::mutex> lk(g_create_mu);
     if (!p->fft) p->fft = new (std::nothrow) pf_fft_cache();
     if (!p->fft) return pf_fail(PF_ERR_ALLOC, "host allocation failed");
     return PF_OK;
 }
 
 static int get_entry(pf_plan* p, int RC, int inverse, pf_fft_entry** out) {
-    // the cache exists from plan creation, so concurrent first calls only
-    // meet under its lock
-    if (!p->fft) {
-        int rc = pf_fft_cache_init(p);
-        if (rc != PF_OK) return rc;
-    }
+    // plans whose operators all run the fused passes have no cache until a
+    // pf_fft stage call; concurrent first calls meet under the creation lock,
+    // then under the cache's
+    const int rc = pf_fft_cache_init(p);
+    if (rc != PF_OK) return rc;
     std::lock_guard<std::mutex> lk(p->fft->mu);
     auto key = std::make_tuple(RC, inverse);
     auto it = p->fft->entries.find(key);
