@@ -1990,14 +1990,23 @@ __device__ __forceinline__ void dft_product(const float* s_d, const float2* s_tw
         }
         // operand row 4 q + r holds line 8 (r / 2) + 2 q + r % 2
         const float* d = s_d + kk * LD + cb * 16 + (r16 & 2) * 4 + (r16 >> 2) * 2 + (r16 & 1);
-        // summed 16 rows at a time and the sums added: the rounding error grows
-        // with sqrt(16 + K / 16) instead of sqrt(K) (K = 200: 2.7 times less)
-        dft_f4 part[MW][4];
-        auto clear = [&]() {
+        // summed 16 rows at a time, those sums 8 at a time, and these added: the
+        // rounding error grows with sqrt(16 + 8 + K / 128) instead of sqrt(K).
+        // 2-D transforms against 64 bits, sums of 16 rows added in one sequence
+        // | so | rocFFT: 484 points 1.64e-7 | 1.50e-7 | 1.59e-7, 880 points 1.86e-7 |
+        // 1.55e-7 | 1.70e-7, 1001 points 1.93e-7 | 1.56e-7 | 1.85e-7
+        dft_f4 sum[MW][4], part[MW][4];
+        auto clear = [&](dft_f4(&v)[MW][4]) {
 #pragma unroll
             for (int q = 0; q < MW; ++q)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) part[q][j] = dft_f4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < 4; ++j) v[q][j] = dft_f4{0.f, 0.f, 0.f, 0.f};
+        };
+        auto add = [&](dft_f4(&v)[MW][4], const dft_f4(&x)[MW][4]) {
+#pragma unroll
+            for (int q = 0; q < MW; ++q)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[q][j] += x[q][j];
         };
         auto step = [&]() {  // 4 rows
             float2 w[MW];
@@ -2017,23 +2026,21 @@ __device__ __forceinline__ void dft_product(const float* s_d, const float2* s_tw
                 part[q][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(bi, w[q].y, part[q][3], 0, 0, 0);
             }
         };
-        auto add = [&]() {
+        for (int k = 0; k < K;) {
+            const int end = min(K, k + 128);
+            clear(sum);
+            for (; k + 16 <= end; k += 16) {
+                clear(part);
 #pragma unroll
-            for (int q = 0; q < MW; ++q)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[q][j] += part[q][j];
-        };
-        int k = 0;
-        for (; k + 16 <= K; k += 16) {
-            clear();
-#pragma unroll
-            for (int st = 0; st < 4; ++st) step();
-            add();
-        }
-        if (k < K) {
-            clear();
-            for (; k < K; k += 4) step();
-            add();
+                for (int st = 0; st < 4; ++st) step();
+                add(sum, part);
+            }
+            if (k < end) {
+                clear(part);
+                for (; k < end; k += 4) step();
+                add(sum, part);
+            }
+            add(acc, sum);
         }
 #pragma unroll
         for (int q = 0; q < MW; ++q) {
