@@ -2026,20 +2026,25 @@ __device__ __forceinline__ void dft_product(const float* s_d, const float2* s_tw
                 part[q][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(bi, w[q].y, part[q][3], 0, 0, 0);
             }
         };
-        for (int k = 0; k < K;) {
+        int k = 0;
+        auto rows = [&](dft_f4(&v)[MW][4]) {  // up to 128 rows into v
             const int end = min(K, k + 128);
-            clear(sum);
             for (; k + 16 <= end; k += 16) {
                 clear(part);
 #pragma unroll
                 for (int st = 0; st < 4; ++st) step();
-                add(sum, part);
+                add(v, part);
             }
             if (k < end) {
                 clear(part);
                 for (; k < end; k += 4) step();
-                add(sum, part);
+                add(v, part);
             }
+        };
+        rows(acc);
+        while (k < K) {
+            clear(sum);
+            rows(sum);
             add(acc, sum);
         }
 #pragma unroll
