@@ -14,9 +14,13 @@
  *     allocating, except the pf_*_create calls, which allocate and
  *     synchronise once when the object is built (fused-FFT twiddle tables
  *     included), so operator calls may be captured into a HIP graph from the
- *     first one.  One exception: grid sizes with prime factors other than
- *     2, 3 and 5 and more than 1024 points run rocFFT, whose plan and work buffer for a new batch size
- *     are made (under the plan's lock) at the first call with that size.
+ *     first one.  One exception: sizes outside 2^a 3^b 5^c and the 7-smooth
+ *     register sizes (pf_pad_fft) that have an axis of more than 1024 points
+ *     run rocFFT, whose plan and work buffer for a new batch size are made
+ *     (under the plan's lock) at the first call with that size.  Such sizes
+ *     with an axis of 400..1024 points run it too for small batches, made at
+ *     the first call outside a capture; a captured first call takes the DFT
+ *     passes instead.  pf_describe_launch says which route a batch takes.
  *   - Every call returns 0 on success or a PF_ERR_* code; pf_last_error()
  *     returns a thread-local message for the last failure.  Arguments are
  *     validated on the host before any launch.
@@ -170,7 +174,9 @@ int pf_nufft_adj(pf_plan* plan, const pf_batch_desc* desc, const void* kspace, v
 
 /* Names of the kernel instances pf_nufft / pf_nufft_adj run for `desc`, as
  * host text "gather=<instance> spread=<instance>[+k_spread_reduce]
- * fft=fused|rocfft" (NUL-terminated, at most cap bytes).  No reference
+ * fft=fused|rocfft[ dft_<axis>=<forward>/<inverse> ...]" (NUL-terminated, at
+ * most cap bytes; dft: lines x output pairs x blocks per group of an axis the
+ * DFT passes transform).  No reference
  * counterpart (the reference's dispatch tables are Python dicts,
  * src/pyfourier/_subroutines/_grid/_cart2noncart/__init__.py:17-18 and
  * _noncart2cart/__init__.py:17-18); lets tests and profiles name what ran. */
@@ -238,12 +244,13 @@ int pf_workspace_offsets(const pf_plan* plan, const pf_batch_desc* desc, size_t*
                          size_t* samples_off, size_t* fft_off, size_t* spread_off);
 
 /* Fused deapodise + zero-pad + centred FFT: image (C, nimg, N...) -> grid.
- * For grid sizes 2^a 3^b 5^c, and the 7-smooth sizes 112, 224, 280, 336 and
- * 448 (<= 4096 per axis), a pruned FFT transforms only the lines that hold
- * image data; other
- * lengths up to 1024 do so with a dense DFT; otherwise pf_deapod_pad +
- * pf_fft.  On the 7-smooth sizes a
- * batch takes at most 16 field-map segments per call.
+ * For grid sizes 2^a 3^b 5^c, and the 7-smooth sizes 56, 112, 168, 224, 280,
+ * 336 and 448 (<= 4096 per axis), a pruned FFT transforms only the lines that
+ * hold image data.  Other lengths up to 1024 do so with a dense DFT, where the
+ * x axis is at most 1024 as well and, from 400 points on, where the batch is
+ * large enough (1 to 16 transforms per call, by length) for it to be the
+ * faster; otherwise pf_deapod_pad + pf_fft.  On the 7-smooth sizes a batch
+ * takes at most 16 field-map segments per call.
  * Replaces src/pyfourier/_nufft/_nufft.py:234-241.  fft_workspace: the FFT
  * scratch part of the pf_nufft workspace (pf_workspace_offsets).  Grid
  * layout (F, C/Cv, G..., nseg*ncoeff, Cv), F = 1 with a basis: Cv is the
@@ -300,7 +307,8 @@ typedef struct pf_toep pf_toep;
  *         needs; copied into the object.  R <= PF_TOEP_RMAX.
  * shape:  host (ndim,) image matrix N (z, y, x).  Embedding sizes 2^a 3^b 5^c
  *         (<= 4096 per axis) and others up to 1024 run the pruned fused FFT
- *         passes, the rest rocFFT. */
+ *         passes, the rest, and small batches of 400 and more points, rocFFT
+ *         (the rule at pf_pad_fft). */
 int pf_toeplitz_create(const void* kernel, int ndim, const int* shape, int nseg, int ncoeff, void* stream,
                        pf_toep** out);
 int pf_toeplitz_destroy(pf_toep* op);
@@ -325,8 +333,7 @@ int pf_toeplitz_apply(pf_toep* op, int batch, const void* image, void* out, cons
  *         (the mask alone without basis and field map); copied.
  * nframes: kernels per image frame (1 with a basis); the image is then
  *         (batch, nframes, N...), or (batch, ncoeff, N...) with a basis.
- * shape:  host (ndim,) N (z, y, x); sizes with prime factors other than 2, 3
- *         and 5 above 1024 use rocFFT. */
+ * shape:  host (ndim,) N (z, y, x); the FFT by the rule at pf_pad_fft. */
 int pf_gram_create(const void* kernel, int ndim, const int* shape, int nframes, int nseg, int ncoeff,
                    void* stream, pf_toep** out);
 
@@ -342,7 +349,8 @@ typedef struct pf_cart pf_cart;
  *        mask; copied.  mframes is 1 (shared by every frame) or the frame
  *        count of the calls.
  * shape: host (ndim,) matrix (z, y, x).  Sizes that factor into 2, 3, 5 use
- *        the fused FFT passes, as do others up to 1024; the rest rocFFT. */
+ *        the fused FFT passes, as do others up to 1024 by the rule at
+ *        pf_pad_fft; the rest rocFFT. */
 int pf_cart_create(const float* mask, int mframes, int ndim, const int* shape, void* stream, pf_cart** out);
 int pf_cart_destroy(pf_cart* plan);
 

@@ -99,16 +99,16 @@ WsLayout layout(const pf_plan* p, const pf_batch& b) {
 
 // FFT state a plan needs before its first operator call: the fused pruned
 // FFT's twiddle tables for the grid sizes it takes (built here, so calls
-// neither allocate nor synchronise), otherwise the rocFFT plan cache, whose
-// per-batch-size rocFFT plans are made on first use under its lock.
+// neither allocate nor synchronise), and where it does not take every batch
+// the rocFFT plan cache, whose per-batch-size rocFFT plans are made on first
+// use under its lock.
 int plan_fft_state(pf_plan* p) {
     int rc = pf_ops_prepare();
     if (rc != PF_OK) return rc;
     // the no-allocation entry point's scratch address on this device; a
     // failure here only disables that entry point (it then reports it)
     if (pf_noalloc_prepare() != PF_OK) pf_set_error("");
-    if (pf_fftk_supported(p)) return pf_fftk_init(p);
-    return pf_fft_cache_init(p);
+    return pf_fft_prepare(p);
 }
 
 }  // namespace
@@ -272,7 +272,7 @@ int pf_describe_launch(const pf_plan* p, const pf_batch_desc* d, char* buf, size
     const std::string spread =
         pf_spread_expand(p, ba, &bx) ? "k_sort_x+" + pf_spread_name(p, bx) : pf_spread_name(p, ba);
     const std::string text = "gather=" + pf_gather_name(p, bf) + " spread=" + spread +
-                             " fft=" + (pf_fftk_supported(p) ? "fused" : "rocfft");
+                             " fft=" + pf_fftk_name(p, bf, ba);
     const size_t n = std::min(cap - 1, text.size());
     std::copy(text.begin(), text.begin() + n, buf);
     buf[n] = 0;
@@ -401,7 +401,7 @@ int pf_pad_fft(pf_plan* p, const pf_batch_desc* d, const void* image, void* grid
     if (rc != PF_OK) return rc;
     if (!image || !grid) return pf_fail(PF_ERR_ARG, "null array");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (pf_fftk_supported(p)) {
+    if (pf_fftk_route(p, b, 0, s)) {
         if (pf_fftk_extra_bytes(p, b) && !fft_workspace) return pf_fail(PF_ERR_ARG, "missing FFT workspace");
         return pf_fftk_forward(p, b, static_cast<const float2*>(image), static_cast<float2*>(grid),
                                static_cast<float2*>(fft_workspace), s);
@@ -418,7 +418,7 @@ int pf_ifft_crop(pf_plan* p, const pf_batch_desc* d, void* grid, void* image, fl
     if (rc != PF_OK) return rc;
     if (!image || !grid) return pf_fail(PF_ERR_ARG, "null array");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (pf_fftk_supported(p)) {
+    if (pf_fftk_route(p, b, 1, s)) {
         if (pf_fftk_extra_bytes(p, b) && !fft_workspace) return pf_fail(PF_ERR_ARG, "missing FFT workspace");
         return pf_fftk_adjoint(p, b, static_cast<float2*>(grid), static_cast<float2*>(image),
                                static_cast<float2*>(fft_workspace), factor, s);
@@ -469,7 +469,7 @@ int pf_run_forward(pf_plan* p, const pf_batch_desc* d, const void* image, void* 
     double factor = 1.0 / p->scale;
     if (norm == PF_NORM_ORTHO) factor /= std::sqrt(ghat(p));
     if (norm == PF_NORM_ADJOINT) factor /= ghat(p);
-    if (pf_fftk_supported(p)) {
+    if (pf_fftk_route(p, b, 0, s)) {
         if ((rc = pf_fftk_forward(p, b, static_cast<const float2*>(image), grid, extra, s)) != PF_OK) return rc;
     } else {
         if ((rc = pf_launch_deapod_pad(p, b, static_cast<const float2*>(image), grid, s)) != PF_OK) return rc;
@@ -501,7 +501,7 @@ int pf_run_adjoint(pf_plan* p, const pf_batch_desc* d, const void* kspace, void*
     // 3-D plans with a column mask: the spread leaves the empty tiles of
     // columns no sample covers unwritten, and the inverse FFT takes those
     // columns as zero without reading them
-    const bool masked = pf_fftk_supported(p) && pf_fftk_masked(p);
+    const bool fused = pf_fftk_route(p, b, 1, s), masked = fused && pf_fftk_masked(p);
     pf_batch bx;
     if (pf_spread_expand(p, b, &bx)) {
         // B0 segments / basis coefficients applied in the sort: a plain spread of R*C items
@@ -515,7 +515,7 @@ int pf_run_adjoint(pf_plan* p, const pf_batch_desc* d, const void* kspace, void*
             return rc;
         if ((rc = pf_launch_spread(p, b, ys, grid, part, s, smax_ready, masked)) != PF_OK) return rc;
     }
-    if (pf_fftk_supported(p))
+    if (fused)
         return pf_fftk_adjoint(p, b, grid, static_cast<float2*>(image), extra, (float)factor, s, masked);
     if ((rc = pf_fft_exec(p, b, grid, 1, s)) != PF_OK) return rc;
     return pf_launch_crop_deapod(p, b, grid, static_cast<float2*>(image), (float)factor, s);

@@ -261,14 +261,12 @@ size_t cart_grid_bytes(const pf_cart* c, const pf_batch& b) {
     return (size_t)b.nfg * b.C * b.R * (size_t)pf_gtot(c->geo) * sizeof(float2);
 }
 
-// mask-only calls on sizes the fused FFT supports run the FFT passes directly
+// mask-only calls the fused FFT takes run the FFT passes directly
 // on the caller's layout (no grid, no transposes, no workspace)
-bool cart_direct(const pf_cart* c, const pf_batch& b) {
-    return b.R == 1 && !b.basis && !b.b0t && pf_fftk_supported(c->geo);
-}
+bool cart_plain(const pf_batch& b) { return b.R == 1 && !b.basis && !b.b0t; }
 
 size_t cart_ws_bytes(const pf_cart* c, const pf_batch& b) {
-    if (cart_direct(c, b)) return 0;
+    if (cart_plain(b) && pf_fftk_use(c->geo, b)) return 0;
     size_t extra = pf_fftk_supported(c->geo) ? pf_fftk_extra_bytes(c->geo, b) : 0;
     return align_up(cart_grid_bytes(c, b)) + align_up(extra);
 }
@@ -378,7 +376,7 @@ int pf_cart_create(const float* mask, int mframes, int ndim, const int* shape, v
     int rc = c->geo ? pf_plan_params(c->geo, ndim, shape, w, sg, 1, 1, nullptr, 0)
                     : pf_fail(PF_ERR_ALLOC, "host allocation failed");
     if (rc == PF_OK) rc = pf_plan_upload_apod(c->geo);
-    if (rc == PF_OK) rc = pf_fftk_supported(c->geo) ? pf_fftk_init(c->geo) : pf_fft_cache_init(c->geo);
+    if (rc == PF_OK) rc = pf_fft_prepare(c->geo);
     if (rc == PF_OK && mask) {
         c->mframes = mframes;
         const size_t n = (size_t)mframes * pf_ntot(c->geo) * sizeof(float);
@@ -427,12 +425,13 @@ int pf_cart_fft(pf_cart* c, const pf_batch_desc* d, int nframes, const void* ima
     double fwd, inv;
     cart_factors(c, norm, &fwd, &inv);
     pf_plan* p = c->geo;
-    if (cart_direct(c, b))
+    const bool fused = pf_fftk_route(p, b, 0, s);
+    if (fused && cart_plain(b))
         return pf_fftk_cart(p, (int64_t)b.C * nframes, nframes, c->mask, c->mframes, true,
                             static_cast<const float2*>(image), static_cast<float2*>(kspace), (float)fwd, s);
     float2* grid = static_cast<float2*>(workspace);
     float2* extra = reinterpret_cast<float2*>(static_cast<char*>(workspace) + align_up(cart_grid_bytes(c, b)));
-    if (pf_fftk_supported(p)) {
+    if (fused) {
         if ((rc = pf_fftk_forward(p, b, static_cast<const float2*>(image), grid, extra, s)) != PF_OK) return rc;
     } else {
         if ((rc = pf_launch_deapod_pad(p, b, static_cast<const float2*>(image), grid, s)) != PF_OK) return rc;
@@ -454,7 +453,8 @@ int pf_cart_ifft(pf_cart* c, const pf_batch_desc* d, int nframes, const void* ks
     double fwd, inv;
     cart_factors(c, norm, &fwd, &inv);
     pf_plan* p = c->geo;
-    if (cart_direct(c, b))
+    const bool fused = pf_fftk_route(p, b, 1, s);
+    if (fused && cart_plain(b))
         return pf_fftk_cart(p, (int64_t)b.C * nframes, nframes, c->mask, c->mframes, false,
                             static_cast<const float2*>(kspace), static_cast<float2*>(image), (float)inv, s);
     float2* grid = static_cast<float2*>(workspace);
@@ -462,7 +462,7 @@ int pf_cart_ifft(pf_cart* c, const pf_batch_desc* d, int nframes, const void* ks
     if ((rc = launch_cart(c, b, nframes, false, nullptr, grid, static_cast<const float2*>(kspace), nullptr, 1.0f, s)) !=
         PF_OK)
         return rc;
-    if (pf_fftk_supported(p))
+    if (fused)
         return pf_fftk_adjoint(p, b, grid, static_cast<float2*>(image), extra, (float)inv, s);
     if ((rc = pf_fft_exec(p, b, grid, 1, s)) != PF_OK) return rc;
     return pf_launch_crop_deapod(p, b, grid, static_cast<float2*>(image), (float)inv, s);

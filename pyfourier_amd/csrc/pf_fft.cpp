@@ -107,6 +107,12 @@ static int get_entry(pf_plan* p, int RC, int inverse, pf_fft_entry** out) {
     return PF_OK;
 }
 
+bool pf_fft_ready(const pf_plan* p, const pf_batch& b, int inverse) {
+    if (!p->fft) return false;
+    std::lock_guard<std::mutex> lk(p->fft->mu);
+    return p->fft->entries.count(std::make_tuple(b.R * b.Cv, inverse)) > 0;
+}
+
 int pf_fft_exec(pf_plan* p, const pf_batch& b, float2* grid, int inverse, hipStream_t stream) {
     const int RC = b.R * b.Cv;
     pf_fft_entry* e = nullptr;

@@ -14,7 +14,7 @@
 //   the X pass writing the deapodised image (sum over B0 segments with the
 //   conjugate maps) in the user layout.
 //
-// Lines of any other length run a pruned DFT on the FP32 matrix cores
+// Lines of other lengths up to 1024 run a pruned DFT on the FP32 matrix cores
 // (k_dftcol, k_dftrow, k_dftcartrow below).  Lines of G = 16 Q points (Q in {5, 6, 7, 8, 9, 10, 12, 14, 15, 16, 18, 20,
 // 21, 24, 25, 28, 30, 32, 36, 40}: 80-640) and of G = 8 Q points (Q in {5,
 // 7, 9, 15, 21, 25, 35, 45}: 40-360) run register four-step kernels: each
@@ -1912,8 +1912,8 @@ __global__ void __launch_bounds__(FT, PF_FFT_WPE) k_cartrow(AxisFFT A, int64_t n
 
 // ---------------------------------------------------------------------------
 // Passes for any other line length G <= DFT_GMAX (a prime factor above 7, or
-// 7 outside the register sizes): the pruned DFT as a product on the FP32
-// matrix cores.  With the line's rows folded about the origin,
+// 7 outside the register sizes; pf_fftk_use says from which batch on): the
+// pruned DFT as a product on the FP32 matrix cores.  With the line's rows folded about the origin,
 // a_k = x_k + x_-k and b_k = x_k - x_-k,
 //
 //     X_m, X_-m = sum_k a_k cos(2 pi k m / G)  -/+  i sum_k b_k sin(2 pi k m / G),
@@ -2370,6 +2370,60 @@ bool pf_fftk_supported(const pf_plan* p) {
     return true;
 }
 
+// lengths rocFFT transforms by radix passes; others it takes through two
+// transforms of more than twice the length
+static bool rocfft_radices(int G) {
+    for (int f : {2, 3, 5, 7, 11, 13, 17})
+        while (G % f == 0) G /= f;
+    return G == 1;
+}
+
+// Transforms per call (planes or volumes: frames x batch x R) from which the DFT
+// passes beat rocFFT with separate pad and crop kernels, by length.  A pass is as
+// long as its longest serial chain of products until the lines fill the chip,
+// so single long planes lose and batches win (rocFFT's strided batches slow
+// down from 16 on).  Measured, us, rocFFT | DFT passes, on either side of each line:
+//   392^2 x 1 34 | 33, x 4 45 | 39;  490^2 x 1 30 | 39, x 2 39 | 40, x 4 61 | 48;
+//   Gram, 490^2 grid x 1 47 | 60, x 4 100 | 75;  572^2 x 4 76 | 72, x 16 414 | 248
+//   616^2 x 4 69 | 95, x 8 146 | 185, x 16 415 | 353;  784^2 x 8 260 | 304, x 16 709 | 774,
+//   x 32 1488 | 1394;  1001^2 x 4 179 | 234, x 16 1220 | 978
+//   fwd + adj, 784^2 grid of 392^2 x 4 180 | 215, x 8 461 | 339;  of 627^2 x 8 481 | 603, x 16 1376 | 1088
+// and where rocFFT has no radix passes
+//   617^2 x 1 64 | 53;  701^2 x 1 67 | 80, x 8 317 | 246;  1021^2 x 4 231 | 237, x 8 564 | 525
+//   fwd + adj, 1002^2 grid of 501^2 x 1 155 | 139;  of 801^2 x 4 429 | 534, x 8 1038 | 965
+static int dft_min_transforms(int G, int N) {
+    if (!rocfft_radices(G)) return G < 650 || N <= 525 ? 1 : 8;
+    if (G < 400) return 1;
+    if (G < 600) return 4;
+    return N <= 525 ? 8 : 16;
+}
+
+bool pf_fftk_use(const pf_plan* p, int64_t transforms) {
+    if (pf_fftk_radix(p)) return true;
+    if (!pf_fftk_supported(p)) return false;
+    if (p->ndim == 1) return true;  // 1001 points x 1 24 | 21, x 4096 628 | 149
+    for (int a = 3 - p->ndim; a < 3; ++a)
+        if (!fftk_axis_ok(p->os[a]) && transforms < dft_min_transforms(p->os[a], p->shape[a])) return false;
+    return true;
+}
+
+bool pf_fftk_route(const pf_plan* p, const pf_batch& b, int inverse, hipStream_t s) {
+    if (pf_fftk_use(p, b)) return true;
+    if (!pf_fftk_supported(p) || pf_fft_ready(p, b, inverse)) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st == hipStreamCaptureStatusActive;
+}
+
+int pf_fft_prepare(pf_plan* p) {
+    if (!pf_fftk_supported(p)) return pf_fft_cache_init(p);
+    const int rc = pf_fftk_init(p);
+    return rc != PF_OK || pf_fftk_use(p, 1) ? rc : pf_fft_cache_init(p);
+}
+
 int pf_fftk_init(pf_plan* p) {
     if (p->fftk) return PF_OK;
     pf_fftk* f = new pf_fftk();
@@ -2552,10 +2606,29 @@ static int dft_shape(const pf_fftk_axis& X, bool fwd, bool split, Blocks&& block
     return PF_OK;
 }
 
+static int dft_col_shape(const pf_fftk_axis& X, bool fwd, bool split, int64_t O, int64_t I, DftShape& d) {
+    return dft_shape(X, fwd, split, [&](int CT) { return O * ((I + CT - 1) / CT); }, d);
+}
+
+// KC values of YG image rows per block, nkc blocks per row group
+static int dft_row_shape(const pf_plan* p, const pf_batch& b, bool fwd, DftShape& d, int& KC, int& YG, int& nkc) {
+    const int KCv = b.K * b.Cv, VT = fwd ? b.L * KCv : KCv;
+    const int64_t rows = (int64_t)b.nfg * b.Cb * p->shape[0] * p->shape[1];
+    return dft_shape(
+        p->fftk->ax[2], fwd, true,
+        [&](int CT) {
+            KC = std::min(VT, CT);
+            YG = CT / KC;
+            nkc = (VT + KC - 1) / KC;
+            return (rows + YG - 1) / YG * nkc;
+        },
+        d);
+}
+
 static int launch_dft_col(const pf_fftk_axis& X, bool fwd, bool cart, int64_t O, int64_t I, const float2* src,
                           float2* dst, const ColMask& cm, const CartEpi& e, hipStream_t s) {
     DftShape d;
-    const int rc = dft_shape(X, fwd, src != dst, [&](int CT) { return O * ((I + CT - 1) / CT); }, d);
+    const int rc = dft_col_shape(X, fwd, src != dst, O, I, d);
     if (rc != PF_OK || d.grid.x < 1) return rc;
 #define PF_DFTCOL(F, T, W, C) \
     hipLaunchKernelGGL((k_dftcol<F, T, W, C>), d.grid, dim3(d.threads), d.lds, s, X.G, X.N, I, X.tw, src, dst, cm, e)
@@ -2582,19 +2655,9 @@ static int launch_dft_col(const pf_fftk_axis& X, bool fwd, bool cart, int64_t O,
 static int launch_dft_row(const pf_plan* p, const pf_batch& b, bool fwd, const float2* src, float2* dst, float factor,
                           hipStream_t s) {
     const pf_fftk_axis& X = p->fftk->ax[2];
-    const int KCv = b.K * b.Cv, VT = fwd ? b.L * KCv : KCv;
-    const int64_t rows = (int64_t)b.nfg * b.Cb * p->shape[0] * p->shape[1];
     int KC = 1, YG = 1, nkc = 1;
     DftShape d;
-    const int rc = dft_shape(
-        X, fwd, true,
-        [&](int CT) {
-            KC = std::min(VT, CT);
-            YG = CT / KC;
-            nkc = (VT + KC - 1) / KC;
-            return (rows + YG - 1) / YG * nkc;
-        },
-        d);
+    const int rc = dft_row_shape(p, b, fwd, d, KC, YG, nkc);
     if (rc != PF_OK || d.grid.x < 1) return rc;
     const Geo g = geo_of(p);
     const Batch t = batch_of(b);
@@ -2617,6 +2680,28 @@ static int launch_dft_row(const pf_plan* p, const pf_batch& b, bool fwd, const f
 #undef PF_DFTROW
     PF_HIP(hipGetLastError());
     return PF_OK;
+}
+
+std::string pf_fftk_name(const pf_plan* p, const pf_batch& bf, const pf_batch& ba) {
+    if (!pf_fftk_use(p, bf)) return "rocfft";
+    std::string name = "fused";
+    if (!p->fftk) return name;
+    for (int a = 3 - p->ndim; a < 3; ++a) {
+        if (!p->fftk->ax[a].dense) continue;
+        name += std::string(" dft_") + "zyx"[a] + "=";
+        for (int inv = 0; inv < 2; ++inv) {
+            const pf_batch& b = inv ? ba : bf;
+            const int64_t FC = (int64_t)b.nfg * b.Cb, row = (int64_t)p->os[2] * b.R * b.Cv;
+            DftShape d{};
+            int KC, YG, nkc;
+            const int rc = a == 2 ? dft_row_shape(p, b, !inv, d, KC, YG, nkc)
+                                  : dft_col_shape(p->fftk->ax[a], !inv, true, a == 0 || p->ndim == 2 ? FC : FC * p->shape[0],
+                                                  a == 0 ? p->os[1] * row : row, d);
+            if (rc == PF_OK)
+                name += (inv ? "/" : "") + std::to_string(d.CT) + "x" + std::to_string(16 * d.MW) + "x" + std::to_string(d.grid.y);
+        }
+    }
+    return name;
 }
 
 static int launch_dft_cartrow(const pf_fftk_axis& X, bool fwd, int64_t nrows, const float2* src, float2* dst,

@@ -140,7 +140,7 @@ struct pf_plan {
     int max_chunk = 0;    // spread entries per work item (0: automatic)
     pf_glist gl;          // LDS-staged gather lists (empty when not built)
 
-    pf_fft_cache* fft = nullptr;   // rocFFT plans (sizes the fused FFT does not take)
+    pf_fft_cache* fft = nullptr;   // rocFFT plans (calls the fused FFT does not take)
     struct pf_fftk* fftk = nullptr; // fused pruned FFT (pf_fftk_supported)
 };
 
@@ -219,6 +219,7 @@ int pf_run_adjoint(pf_plan* p, const pf_batch_desc* d, const void* kspace, void*
                    void* workspace, size_t workspace_bytes, void* stream, bool lean);
 int pf_launch_sort_expand(const pf_plan* p, const pf_batch& b, const float2* y, float2* ys, const float* weight,
                           hipStream_t s);
+bool pf_fft_ready(const pf_plan* p, const pf_batch& b, int inverse);  // the rocFFT plan of this batch is made
 int pf_fft_exec(pf_plan* p, const pf_batch& b, float2* grid, int inverse, hipStream_t s);
 void pf_fft_destroy(pf_fft_cache* c);
 int pf_fft_cache_init(pf_plan* p);  // rocFFT setup + the plan's (empty) cache
@@ -236,6 +237,16 @@ int pf_noalloc_prepare();  // this device's pf_nufft_noalloc scratch address, at
 // fused deapodise/pad/FFT and inverse FFT/crop/deapodise (pf_fftk.hip)
 bool pf_fftk_supported(const pf_plan* p);
 bool pf_fftk_radix(const pf_plan* p);  // by the radix and register passes alone
+// whether a call of that many transforms runs the fused passes: long lengths
+// outside the radix sets run rocFFT for a few
+bool pf_fftk_use(const pf_plan* p, int64_t transforms);
+static inline bool pf_fftk_use(const pf_plan* p, const pf_batch& b) { return pf_fftk_use(p, (int64_t)b.nfg * b.C * b.R); }
+// the same for a call on a stream: under capture, where nothing may be allocated,
+// a call whose rocFFT plan is not made yet runs the fused passes too
+bool pf_fftk_route(const pf_plan* p, const pf_batch& b, int inverse, hipStream_t s);
+int pf_fft_prepare(pf_plan* p);  // the FFT state a plan's calls need, at its creation
+// a call's FFT path (batches of the forward and the adjoint)
+std::string pf_fftk_name(const pf_plan* p, const pf_batch& bf, const pf_batch& ba);
 int pf_fftk_init(pf_plan* p);
 int pf_fftk_ready(const pf_plan* p);  // PF_OK when pf_fftk_init has run
 void pf_fftk_destroy(struct pf_fftk* f);

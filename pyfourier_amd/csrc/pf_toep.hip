@@ -154,7 +154,7 @@ int toep_create(const void* kernel, int ndim, const int* shape, int nfr, int nse
     float s[3] = {sigma, sigma, sigma};
     int rc = t->geo ? pf_plan_params(t->geo, ndim, shape, w, s, 1, 1, nullptr, 0) : pf_fail(PF_ERR_ALLOC, "host allocation");
     if (rc == PF_OK) rc = pf_plan_upload_apod(t->geo);
-    if (rc == PF_OK) rc = pf_fftk_supported(t->geo) ? pf_fftk_init(t->geo) : pf_fft_cache_init(t->geo);
+    if (rc == PF_OK) rc = pf_fft_prepare(t->geo);
     if (rc == PF_OK) {
         const size_t n = (size_t)nfr * pf_gtot(t->geo) * R * R * sizeof(float2);
         hipError_t e = hipMalloc(&t->T, n);
@@ -215,15 +215,14 @@ int pf_toeplitz_apply(pf_toep* t, int batch, const void* image, void* out, const
     hipStream_t s = static_cast<hipStream_t>(stream);
     float2* grid = static_cast<float2*>(workspace);
     float2* extra = reinterpret_cast<float2*>(static_cast<char*>(workspace) + gb);
-    const bool fused = pf_fftk_supported(t->geo);
     if (pf_fftk_gram_supported(t->geo, b))
         return pf_fftk_gram(t->geo, b, static_cast<const float2*>(image), static_cast<float2*>(out), grid, extra, t->T,
                             (float)(1.0 / (double)pf_gtot(t->geo)), s);
     int rc;
-    if (fused) {
+    if (pf_fftk_route(t->geo, b, 0, s)) {
         rc = pf_fftk_forward(t->geo, b, static_cast<const float2*>(image), grid, extra, s);
     } else {
-        // sizes the fused FFT does not take: generic pad, rocFFT, crop
+        // calls the fused FFT does not take: generic pad, rocFFT, crop
         rc = pf_launch_deapod_pad(t->geo, b, static_cast<const float2*>(image), grid, s);
         if (rc == PF_OK) rc = pf_fft_exec(t->geo, b, grid, 0, s);
     }
@@ -245,7 +244,7 @@ int pf_toeplitz_apply(pf_toep* t, int batch, const void* image, void* out, const
     }
     PF_HIP(hipGetLastError());
     const float factor = (float)(1.0 / (double)gtot);
-    if (fused) return pf_fftk_adjoint(t->geo, b, grid, static_cast<float2*>(out), extra, factor, s);
+    if (pf_fftk_route(t->geo, b, 1, s)) return pf_fftk_adjoint(t->geo, b, grid, static_cast<float2*>(out), extra, factor, s);
     if ((rc = pf_fft_exec(t->geo, b, grid, 1, s)) != PF_OK) return rc;
     return pf_launch_crop_deapod(t->geo, b, grid, static_cast<float2*>(out), factor, s);
 }
