@@ -252,7 +252,8 @@ int pf_workspace_offsets(const pf_plan* plan, const pf_batch_desc* desc, size_t*
  * faster; otherwise pf_deapod_pad + pf_fft.  On the 7-smooth sizes a batch
  * takes at most 16 field-map segments per call.
  * Replaces src/pyfourier/_nufft/_nufft.py:234-241.  fft_workspace: the FFT
- * scratch part of the pf_nufft workspace (pf_workspace_offsets).  Grid
+ * scratch part of the pf_nufft workspace (pf_workspace_offsets); NULL makes
+ * sizes outside the first two kinds take pf_deapod_pad + pf_fft.  Grid
  * layout (F, C/Cv, G..., nseg*ncoeff, Cv), F = 1 with a basis: Cv is the
  * largest divisor of C up to 64, or 2 (coil pairs) for a 3-D plan with one
  * kernel width of 3..8 on all axes and an even C with no field map or basis. */

@@ -111,6 +111,12 @@ int plan_fft_state(pf_plan* p) {
     return pf_fft_prepare(p);
 }
 
+// FFT stage calls: without a workspace, sizes outside the radix sets take the
+// in-place rocFFT stage, which needs none
+bool stage_fused(const pf_plan* p, const pf_batch& b, int inverse, const void* fft_workspace, hipStream_t s) {
+    return pf_fftk_route(p, b, inverse, s) && (pf_fftk_radix(p) || fft_workspace || !pf_fftk_extra_bytes(p, b));
+}
+
 }  // namespace
 
 // Deapodisation vectors per axis (src/pyfourier/_subroutines/_apod.py:27-41):
@@ -401,7 +407,7 @@ int pf_pad_fft(pf_plan* p, const pf_batch_desc* d, const void* image, void* grid
     if (rc != PF_OK) return rc;
     if (!image || !grid) return pf_fail(PF_ERR_ARG, "null array");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (pf_fftk_route(p, b, 0, s)) {
+    if (stage_fused(p, b, 0, fft_workspace, s)) {
         if (pf_fftk_extra_bytes(p, b) && !fft_workspace) return pf_fail(PF_ERR_ARG, "missing FFT workspace");
         return pf_fftk_forward(p, b, static_cast<const float2*>(image), static_cast<float2*>(grid),
                                static_cast<float2*>(fft_workspace), s);
@@ -418,7 +424,7 @@ int pf_ifft_crop(pf_plan* p, const pf_batch_desc* d, void* grid, void* image, fl
     if (rc != PF_OK) return rc;
     if (!image || !grid) return pf_fail(PF_ERR_ARG, "null array");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (pf_fftk_route(p, b, 1, s)) {
+    if (stage_fused(p, b, 1, fft_workspace, s)) {
         if (pf_fftk_extra_bytes(p, b) && !fft_workspace) return pf_fail(PF_ERR_ARG, "missing FFT workspace");
         return pf_fftk_adjoint(p, b, static_cast<float2*>(grid), static_cast<float2*>(image),
                                static_cast<float2*>(fft_workspace), factor, s);

@@ -107,3 +107,11 @@ def test_cartesian_instances(cuda_device, shape, C):
     for a, r in ((y, yr), (z, zr)):
         a = a.cpu().reshape(r.shape)
         assert float((a - r).norm() / r.norm()) < STAGE
+
+
+def test_stages_without_a_workspace(cuda_device):
+    """Sizes outside the radix sets take a null FFT workspace (the in-place
+    stage); the radix sizes refuse it."""
+    _stages(cuda_device, (37, 29), 1.5, 3, "fft=fused", workspace=False)
+    with pytest.raises(RuntimeError, match="missing FFT workspace"):
+        _stages(cuda_device, (32, 32), 2.0, 3, "fft=fused", workspace=False)
