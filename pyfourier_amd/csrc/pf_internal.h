@@ -66,9 +66,6 @@ struct pf_slist {
 #ifndef PF_COLMASK
 #define PF_COLMASK 1  // 3-D plans: skip the (y, x) grid columns no sample covers in the fused operators
 #endif
-#ifndef PF_SPREAD_MINCH
-#define PF_SPREAD_MINCH 64  // smallest work item of the fine split (entries)
-#endif
 
 
 // Gather column lists (3-D plans with one kernel width on all axes): the

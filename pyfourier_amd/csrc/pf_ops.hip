@@ -420,7 +420,7 @@ __global__ void __launch_bounds__(GCOL_TB, 2)
     const float4* pairs = reinterpret_cast<const float4*>(grid) + (int64_t)(B.nfg > 1 ? f : 0) * B.Cb * g.gtot;
     const int tid = threadIdx.x, wave = tid >> 6;
 
-    // this thread's staged points p = tid, tid + 256, ...: their grid point
+    // this thread's staged points p = tid, tid + GCOL_TB, ...: their grid point
     // index (periodic wrap), -1 past the window
     int goff[S::NK];
 #pragma unroll
@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(GCOL_TB, 2)
     // written far apart in time (each a partial cache-line write to HBM)
     float4 o[GCOL_OUT];
     for (int cp = 0; cp < ncp; ++cp) {
-        // window -> LDS: lane i of wave w, copy k lands at point k*256 + w*64 + i
+        // window -> LDS: lane i of wave w, copy k lands at point k*GCOL_TB + w*64 + i
         const float4* pair = pairs + (int64_t)cp * g.gtot;
 #pragma unroll
         for (int k = 0; k < S::NK; ++k)
@@ -1011,7 +1011,7 @@ __global__ void __launch_bounds__(64, spread_wreg<100 * TZ + TY>() ? 3 : 1) k_sp
 // point and writes 16 bytes.  Measured (spread kernel alone, before -> after):
 // 3-D 256^3 grid x 8 coils, 2.1M samples, W = 4 983 -> 414 us (its 1.1 GB of
 // grid alone takes 220 us at the 4.9 TB/s of a copy); 113 x 128 x 138 grid x 6
-// coils, 660k samples 1080 -> 232 us; 2-D 320^2 x 16 coils, 197k samples 77 ->
+// coils, 660k samples 1080 -> 120 us; 2-D 320^2 x 16 coils, 197k samples 77 ->
 // 34 us; 512^2 x 32 values, 1M samples 421 -> 210 us; 256^2 x 1 coil, 16k
 // samples 24.5 -> 6.1 us.
 // -------------------------------------------------------------------------
@@ -1253,9 +1253,9 @@ __global__ void __launch_bounds__(64, VL == 32 ? 2 : (VL == 16 ? 3 : 4))
 }
 
 // -------------------------------------------------------------------------
-// Matrix-core spread: the same items, entry batches, copies and summation
-// order over batches as k_spread_pipe, with the accumulation of a batch done
-// by MFMA.  For a batch of SPIPE_EB = 16 entries the tile update is a product
+// fp16-split matrix-core spread: the same items, entry batches and summation
+// order over batches as k_spread_pipe; records and values are copied global ->
+// LDS two batches ahead.  The accumulation of a batch is done by fp16 MFMA.  For a batch of SPIPE_EB = 16 entries the tile update is a product
 //
 //     acc[p, n] += sum_k A[p, k] * B[k, n],   A[p, k] = wz * wy * wx of entry k
 //                                             at tile point p (0 outside its

@@ -47,7 +47,7 @@ CASES = [
     ("3d_basis", (12, 10, 16), 2, 6, 6, 2, None),
     ("1d", (50,), 4, 1, 1, 0, None),
     ("odd_sizes", (45, 75), 2, 1, 1, 0, None),
-    ("rocfft_sizes", (14, 22), 3, 2, 2, 0, "ortho"),
+    ("dft_sizes", (14, 22), 3, 2, 2, 0, "ortho"),
     ("rows_256", (256, 256), 2, 1, 1, 0, None),
     ("many_coils", (16, 64), 96, 1, 1, 0, None),
     ("coil_blocks", (8, 40), 130, 2, 2, 0, "ortho"),

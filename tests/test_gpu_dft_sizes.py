@@ -1,6 +1,7 @@
 """Grid and matrix sizes with prime factors outside the radix sets: the DFT
 passes on the matrix cores, as rows and columns, forward and inverse, at the
-edges of their tiles (16 and 32 lines, 32 output pairs, 4 folded rows)."""
+edges of the tiles that few lines take (16 lines, 16 output pairs, 4 folded
+rows) and, in the volumes, 32 lines.  test_gpu_dft_shapes.py has the others."""
 
 import numpy as np
 import pytest

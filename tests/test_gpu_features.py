@@ -56,8 +56,9 @@ def test_3d_anisotropic(cuda_device):
     _check_pair(cuda_device, coord, shape, x, width=(4, 5, 6), oversamp=(2.0, 1.5, 1.25))
 
 
-def test_rocfft_fallback_size(cuda_device):
-    # oversampled size 147 = 3 * 7^2 is outside the fused FFT's radix set
+def test_size_outside_the_radix_set(cuda_device):
+    # oversampled size 147 = 3 * 7^2: the matrix-core DFT passes (the rocFFT
+    # route has its own cases in test_gpu_dft_rule.py)
     rng = np.random.default_rng(2)
     coord = demo.golden_angle_radial_2d(40, 120)
     x = demo.complex_gaussian(rng, (2, 98, 98))
