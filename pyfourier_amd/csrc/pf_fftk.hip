@@ -2382,9 +2382,12 @@ static bool rocfft_radices(int G) {
 // passes beat rocFFT with separate pad and crop kernels, by length.  A pass is as
 // long as its longest serial chain of products until the lines fill the chip,
 // so single long planes lose and batches win (rocFFT's strided batches slow
-// down from 16 on).  Measured, us, rocFFT | DFT passes, on either side of each line:
-//   392^2 x 1 34 | 33, x 4 45 | 39;  490^2 x 1 30 | 39, x 2 39 | 40, x 4 61 | 48;
-//   Gram, 490^2 grid x 1 47 | 60, x 4 100 | 75;  572^2 x 4 76 | 72, x 16 414 | 248
+// down from 16 on).  rocFFT also makes a plan at the first call with a batch
+// size, 9 ms against 0.25 ms, which a gain of a few us does not earn back: the
+// shortest line lies where single planes lose 10 us.  Measured, us a call, rocFFT |
+// DFT passes, on either side of each line:
+//   392^2 x 1 34 | 33;  490^2 x 1 33 | 39, x 2 39 | 40, x 4 61 | 48;  Gram, 490^2 grid x 1 47 | 60,
+//   x 2 65 | 66;  572^2 x 1 34 | 48, x 2 53 | 54, x 4 76 | 72, x 16 414 | 248
 //   616^2 x 4 69 | 95, x 8 146 | 185, x 16 415 | 353;  784^2 x 8 260 | 304, x 16 709 | 774,
 //   x 32 1488 | 1394;  1001^2 x 4 179 | 234, x 16 1220 | 978
 //   fwd + adj, 784^2 grid of 392^2 x 4 180 | 215, x 8 461 | 339;  of 627^2 x 8 481 | 603, x 16 1376 | 1088
@@ -2393,8 +2396,8 @@ static bool rocfft_radices(int G) {
 //   fwd + adj, 1002^2 grid of 501^2 x 1 155 | 139;  of 801^2 x 4 429 | 534, x 8 1038 | 965
 static int dft_min_transforms(int G, int N) {
     if (!rocfft_radices(G)) return G < 650 || N <= 525 ? 1 : 8;
-    if (G < 400) return 1;
-    if (G < 600) return 4;
+    if (G < 500) return 1;
+    if (G < 600) return 2;
     return N <= 525 ? 8 : 16;
 }
 
