@@ -18,9 +18,9 @@
  *     register sizes (pf_pad_fft) that have an axis of more than 1024 points
  *     run rocFFT, whose plan and work buffer for a new batch size are made
  *     (under the plan's lock) at the first call with that size.  Such sizes
- *     with an axis of 500..1024 points run it too for small batches, made at
- *     the first call outside a capture; a captured first call takes the DFT
- *     passes instead.  pf_describe_launch says which route a batch takes.
+ *     up to 1024 with more than 525 image points along an axis run it too for
+ *     small batches, made at the first call outside a capture; a captured first
+ *     call takes the DFT passes instead.  pf_describe_launch says which route a batch takes.
  *   - Every call returns 0 on success or a PF_ERR_* code; pf_last_error()
  *     returns a thread-local message for the last failure.  Arguments are
  *     validated on the host before any launch.
@@ -247,9 +247,9 @@ int pf_workspace_offsets(const pf_plan* plan, const pf_batch_desc* desc, size_t*
  * For grid sizes 2^a 3^b 5^c, and the 7-smooth sizes 56, 112, 168, 224, 280,
  * 336 and 448 (<= 4096 per axis), a pruned FFT transforms only the lines that
  * hold image data.  Other lengths up to 1024 do so with a dense DFT, where the
- * x axis is at most 1024 as well and, from 500 points on, where the batch is
- * large enough (1 to 16 transforms per call, by length) for it to be the
- * faster; otherwise pf_deapod_pad + pf_fft.  On the 7-smooth sizes a batch
+ * x axis is at most 1024 as well and, with more than 525 image points along an
+ * axis, where the batch is large enough (1 to 16 transforms per call, by
+ * length) for it to be the faster; otherwise pf_deapod_pad + pf_fft.  On the 7-smooth sizes a batch
  * takes at most 16 field-map segments per call.
  * Replaces src/pyfourier/_nufft/_nufft.py:234-241.  fft_workspace: the FFT
  * scratch part of the pf_nufft workspace (pf_workspace_offsets); NULL makes
@@ -308,8 +308,7 @@ typedef struct pf_toep pf_toep;
  *         needs; copied into the object.  R <= PF_TOEP_RMAX.
  * shape:  host (ndim,) image matrix N (z, y, x).  Embedding sizes 2^a 3^b 5^c
  *         (<= 4096 per axis) and others up to 1024 run the pruned fused FFT
- *         passes, the rest, and small batches of 500 and more points, rocFFT
- *         (the rule at pf_pad_fft). */
+ *         passes, the rest rocFFT (the rule at pf_pad_fft). */
 int pf_toeplitz_create(const void* kernel, int ndim, const int* shape, int nseg, int ncoeff, void* stream,
                        pf_toep** out);
 int pf_toeplitz_destroy(pf_toep* op);

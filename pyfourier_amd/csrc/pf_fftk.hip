@@ -2379,26 +2379,24 @@ static bool rocfft_radices(int G) {
 }
 
 // Transforms per call (planes or volumes: frames x batch x R) from which the DFT
-// passes beat rocFFT with separate pad and crop kernels, by length.  A pass is as
-// long as its longest serial chain of products until the lines fill the chip,
-// so single long planes lose and batches win (rocFFT's strided batches slow
-// down from 16 on).  rocFFT also makes a plan at the first call with a batch
-// size, 9 ms against 0.25 ms, which a gain of a few us does not earn back: the
-// shortest line lies where single planes lose 10 us.  Measured, us a call, rocFFT |
-// DFT passes, on either side of each line:
-//   392^2 x 1 34 | 33;  490^2 x 1 33 | 39, x 2 39 | 40, x 4 61 | 48;  Gram, 490^2 grid x 1 47 | 60,
-//   x 2 65 | 66;  572^2 x 1 34 | 48, x 2 53 | 54, x 4 76 | 72, x 16 414 | 248
-//   616^2 x 4 69 | 95, x 8 146 | 185, x 16 415 | 353;  784^2 x 8 260 | 304, x 16 709 | 774,
-//   x 32 1488 | 1394;  1001^2 x 4 179 | 234, x 16 1220 | 978
-//   fwd + adj, 784^2 grid of 392^2 x 4 180 | 215, x 8 461 | 339;  of 627^2 x 8 481 | 603, x 16 1376 | 1088
-// and where rocFFT has no radix passes
-//   617^2 x 1 64 | 53;  701^2 x 1 67 | 80, x 8 317 | 246;  1021^2 x 4 231 | 237, x 8 564 | 525
-//   fwd + adj, 1002^2 grid of 501^2 x 1 155 | 139;  of 801^2 x 4 429 | 534, x 8 1038 | 965
+// passes beat rocFFT with separate pad and crop kernels, by the grid and image
+// length.  A pass is as long as its longest serial chain of products until the
+// lines fill the chip, so single long planes lose and batches win (rocFFT's
+// strided batches slow down from 16 on).  rocFFT also makes a plan at the first
+// call with a batch size, 9 to 20 ms a direction against none here, which a few
+// tens of us a call earn back only after hundreds of calls: lengths with up to
+// 525 image points keep the DFT passes at any batch.  Measured, us, rocFFT | DFT:
+//   up to 525: 490^2 x 1 33 | 39, x 4 61 | 48;  Gram, 490^2 grid x 1 47 | 60, x 2 65 | 66;  784^2 x 1
+//   70 | 98, x 8 456 | 322;  fwd + adj, 704^2 grid of 352^2 x 1 78 | 96, x 2 104 | 122, x 8 375 | 259
+//   longer: 572^2 x 1 34 | 48, x 2 53 | 54, x 4 76 | 72;  616^2 x 8 146 | 185, x 16 415 | 353;
+//   784^2 x 1 47 | 106, x 8 260 | 304, x 16 709 | 774, x 32 1488 | 1394;  1001^2 x 1 59 | 144, x 16
+//   1220 | 978;  fwd + adj, 784^2 grid of 627^2 x 8 481 | 603, x 16 1376 | 1088
+//   and where rocFFT has no radix passes: 617^2 x 1 64 | 53;  701^2 x 1 67 | 80, x 8 317 | 246;
+//   1021^2 x 4 231 | 237, x 8 564 | 525;  fwd + adj, 1002^2 grid of 801^2 x 4 429 | 534, x 8 1038 | 965
 static int dft_min_transforms(int G, int N) {
-    if (!rocfft_radices(G)) return G < 650 || N <= 525 ? 1 : 8;
-    if (G < 500) return 1;
-    if (G < 600) return 2;
-    return N <= 525 ? 8 : 16;
+    if (N <= 525) return 1;
+    if (!rocfft_radices(G)) return G < 650 ? 1 : 8;
+    return G < 600 ? 2 : 16;
 }
 
 bool pf_fftk_use(const pf_plan* p, int64_t transforms) {

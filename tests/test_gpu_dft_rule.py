@@ -1,5 +1,5 @@
 """Which route a length outside the radix sets takes: the matrix-core DFT passes,
-or rocFFT with pad and crop kernels for few transforms of 500 and more points,
+or rocFFT with pad and crop kernels for few transforms of more than 525 image points,
 beyond 1024 points and where the x axis is longer.  Both sides of each line
 against 64-bit results."""
 
@@ -45,14 +45,14 @@ def _nufft(dev, shape, oversamp, C, route):
         ((308, 10), 1.25, 1),   # 385 points: always the DFT passes
         ((314, 10), 1.25, 1),   # 393 = 3 * 131: no radix passes in rocFFT
         ((392, 10), 1.25, 1),   # 490
-        ((457, 10), 1.25, 2),   # 572
-        ((10, 457), 1.25, 2),
-        ((352, 8), 2.0, 8),     # 704 of 352
+        ((526, 10), 1.13, 2),   # 595
+        ((10, 526), 1.13, 2),
+        ((352, 8), 2.0, 1),     # 704 of 352
         ((563, 8), 1.25, 16),   # 704 of 563
         ((493, 8), 1.25, 1),    # 617, prime
         ((501, 6), 2.0, 1),     # 1002 = 6 * 167 of 501
         ((550, 8), 1.25, 8),    # 688 = 16 * 43 of 550
-        ((8, 6, 457), 1.25, 2),
+        ((8, 6, 526), 1.13, 2),
     ],
 )
 def test_route_by_batch(cuda_device, shape, oversamp, few):
@@ -104,7 +104,7 @@ def test_toeplitz_embedding(cuda_device, shape, C):
     assert rel(y, ref) < PARITY
 
 
-@pytest.mark.parametrize("shape,oversamp,C", [((457, 10), 1.25, 1), ((563, 8), 1.25, 3)])
+@pytest.mark.parametrize("shape,oversamp,C", [((526, 10), 1.13, 1), ((563, 8), 1.25, 3)])
 def test_first_call_under_capture(cuda_device, shape, oversamp, C):
     """A batch that runs rocFFT may be captured from its first call on: nothing
     is allocated there, so the DFT passes take it; after an eager call the

@@ -1,7 +1,8 @@
 """The FP32 matrix-core spread (k_spread_pipe) at the edges of its forms: each
 values-per-wave instance and its remainders, batches stored as one value per
-grid block, grids smaller than a tile or cut by its edge, every kernel width
-end, split tiles, and frames sharing one grid through a basis of odd size."""
+grid block, grids smaller than a tile or cut by its edge, wide kernels and those
+whose tap records are shorter than the four pieces a wave stages at a time, split
+tiles, and frames sharing one grid through a basis of odd size."""
 
 import numpy as np
 import pytest
@@ -58,6 +59,13 @@ def test_small_grids_and_widths(cuda_device, ndim, shape, width):
         # a grid axis too short for tile + width becomes one tile, which may
         # exceed every instance (the LDS-staged spread then runs)
         _check(cuda_device, ndim, shape, C, width, 2.0, 0, routed=False)
+
+
+@pytest.mark.parametrize("C", [1, 8, 17])
+@pytest.mark.parametrize("ndim,shape,width", [(1, (60,), 2), (1, (60,), 6), (2, (40, 44), 2), (2, (40, 44), 3),
+                                              (3, (24, 20, 26), 2)])  # records of 2 and 3 pieces
+def test_short_records(cuda_device, ndim, shape, width, C):
+    _check(cuda_device, ndim, shape, C, width, 2.0, 0)
 
 
 @pytest.mark.parametrize("C,K", [(5, 3), (1, 3), (3, 7)])
