@@ -441,8 +441,9 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
     // 3-D 2.8M x 8 256, 8.8M x 8 512, 17M x 32 1024).  Never above four times
     // the mean of a non-empty tile (at least 128) or 1024; ordinary tiles are
     // split too where the minimum lies below their entries.  The last split,
-    // for calls short of workspace, takes that upper bound itself; plans too
-    // large for the fixed workspace of such calls share the one before.
+    // for calls short of workspace, takes that upper bound itself; lists whose
+    // grids alone exceed the fixed workspace of such calls share the one before
+    // (no such call can run on them, and hundreds of frames make many items).
     int CH[PF_NSPLIT];
     int64_t nonempty = 0;
     for (uint64_t k = 0; k < nkeys; ++k) nonempty += he[k] > hs[k];
@@ -453,7 +454,7 @@ static int build_slist(pf_plan* p, const TapParams& P, int merge, hipStream_t st
         const int64_t step = (int64_t)std::lround(64.0 * std::exp2(0.5 * std::floor(2.0 * std::log2(std::max(1.0, n / 64.0)) + 0.5)));
         CH[m] = p->max_chunk > 0 ? p->max_chunk : (int)std::min<int64_t>(1024, std::min(heavy, step));
         if (m == PF_NSPLIT - 1 && p->max_chunk <= 0)
-            CH[m] = (size_t)(pf_gtot(p) + p->mtot) * sizeof(float2) <= PF_NOALLOC_SCRATCH_BYTES
+            CH[m] = (size_t)((merge ? 1 : p->nframes) * pf_gtot(p) + p->mtot) * sizeof(float2) <= PF_NOALLOC_SCRATCH_BYTES
                         ? (int)std::min<int64_t>(1024, heavy)
                         : CH[m - 1];
     }
